@@ -22,7 +22,7 @@
  *  - Device entry points take device pointers and a hipStream_t passed as `void*` (NULL = the
  *    null stream).  They are asynchronous and stream-ordered, like the CUDA backend's matmulS
  *    launch (cuda/src/cuda_backend.cu:1534-1542).  They allocate no device memory, except
- *    qvx_qgemm_f16, qvx_gemm16, the many-vector form of qvx_qmatmul_n and the unfused norm route,
+ *    qvx_qgemm_f16, qvx_gemm16, the many-vector forms of qvx_qmatmul_n and the unfused norm route,
  *    which take stream-ordered temporaries (the converted activations, the partial tiles of a K
  *    split, or the dequantised weight) from a memory pool the library owns per device.  Each stream
  *    keeps its last temporary for its next call (no pool call between back-to-back calls), and a
@@ -120,7 +120,12 @@ int qvx_qmatmul(float* d_out, const void* d_w, uint32_t type, const float* d_x, 
  * the VALU kernel, four vectors a launch) and adds them in a second launch.  A plan gives these calls
  * a workspace of its own, allocated by qvx_plan_instantiate, so its replays allocate nothing; on
  * shallow grids (<= 8 vectors, at most two 32-row tiles a workgroup) it also gives the call one
- * zeroed counter a 32-row tile, with which the kernel adds the block sums itself. */
+ * zeroed counter a 32-row tile, with which the kernel adds the block sums itself.
+ * Q8_0 / Q4_0 / Q5_0 batches of 9 vectors or more (of 5 on weights of >= 32 Mi elements, 16 Mi for the 4-
+ * and 5-bit formats), on the one-vector kernel's shapes, run on a matrix-core form that converts the
+ * activations once into a stream-ordered temporary (n_vec * cols * 2.06 bytes, at most about 64 MiB: larger
+ * batches run in parts) or a plan's workspace, and reads the weights once per 16 to 64 vectors; on a
+ * capturing stream they keep the one-vector kernel's launches, which take no temporary. */
 int qvx_qmatmul_n(float* d_out, const void* d_w, uint32_t type, const float* d_X, int n_vec,
                   int rows, int cols, void* stream);
 

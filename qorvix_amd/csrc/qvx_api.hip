@@ -68,6 +68,10 @@ size_t gemv_many_ws_bytes(int nvec, int rows, int cols, size_t row_bytes);
 int gemv_many_supported(int cols, size_t row_bytes);
 bool launch_gemv_q4k_many(const void* w, const float* X, float* Y, const float* bias, int nvec, int rows, int cols,
                           size_t row_bytes, void* ws, hipStream_t s);
+size_t gemv_int_ws_bytes(uint32_t t, int nvec, int rows, int cols, size_t row_bytes);
+bool launch_gemv_int(uint32_t t, const void* w, const float* X, float* Y, const float* bias, int nvec, int rows,
+                     int cols, size_t row_bytes, void* ws, hipStream_t s);
+bool stream_capturing(hipStream_t s);
 void launch_add_bias(float* out, const float* bias, int nvec, int rows, hipStream_t s);
 }  // namespace qvx
 
@@ -238,11 +242,15 @@ inline bool q6_norm_batched(int nvec, int rows, int cols) {
 }
 
 // The forms that take a workspace, and the bytes of the one a call takes (0: none).
-enum WsForm { WS_NONE, WS_MANY, WS_Q4S, WS_Q6S, WS_Q6S_NORM };
+enum WsForm { WS_NONE, WS_MANY, WS_Q4S, WS_Q6S, WS_Q6S_NORM, WS_INT };
 inline WsForm ws_route(uint32_t type, int nvec, int rows, int cols, size_t row_bytes, bool fast, const GemvEpi& epi,
                        size_t* bytes) {
   *bytes = 0;
   if (!fast || rows <= 0 || cols <= 0) return WS_NONE;
+  if (!epi.flags()) {
+    *bytes = gemv_int_ws_bytes(type, nvec, rows, cols, row_bytes);
+    if (*bytes) return WS_INT;
+  }
   if (epi.flags()) {
     if (type == T_Q6_K && epi.flags() == EPI_NORM && q6_norm_batched(nvec, rows, cols) &&
         gemv_fast_fusable(type, cols, row_bytes, epi) && gemv_q6s_route(nvec, rows, cols, row_bytes, bytes)) {
@@ -294,12 +302,16 @@ int gemv(float* out, const void* w, uint32_t type, const float* X, int nvec, int
   //    per vector to the one-vector kernel, the bias added in its sum launch;
   //  * Q6_K batches (q6_batched): the matrix-core form with the K range split over workgroups
   //    (k_gemv_q6s), bit-identical per vector to the VALU kernel; a bias is added after;
+  //  * Q8_0 / Q4_0 / Q5_0 batches: activations converted once, then the matrix-core form with the VALU
+  //    kernel's arithmetic (k_gemv_int), the bias in its store; a capturing stream keeps the VALU kernel
+  //    (the same bits), so that a captured call takes no temporary;
   //  * Q6_K batches with the RMSNorm prologue (q6_norm_batched): the standalone norm into the
   //    workspace, then that form on the normalised activations.
   size_t need = 0;
   if (const WsForm form = ws_route(type, nvec, rows, cols, row_bytes, fast, epi, &need); form != WS_NONE) {
     const bool own = epi.ws && epi.ws_bytes >= need;
-    void* ws = own ? epi.ws : epi.no_alloc ? nullptr : gemm_temp_alloc(need, s);
+    const bool none = epi.no_alloc || (form == WS_INT && !own && stream_capturing(s));
+    void* ws = own ? epi.ws : none ? nullptr : gemm_temp_alloc(need, s);
     if (ws) {
       uint32_t* cnt = own && epi.cnt_n >= gemv_q6s_counters(nvec, rows, cols) ? epi.cnt : nullptr;
       bool ok;
@@ -311,6 +323,7 @@ int gemv(float* out, const void* w, uint32_t type, const float* X, int nvec, int
                              s, cnt);
       } else {
         ok = form == WS_MANY ? launch_gemv_q4k_many(w, X, out, epi.bias, nvec, rows, cols, row_bytes, ws, s)
+             : form == WS_INT ? launch_gemv_int(type, w, X, out, epi.bias, nvec, rows, cols, row_bytes, ws, s)
              : form == WS_Q4S ? launch_gemv_q4s(w, X, out, epi.bias, nvec, rows, cols, row_bytes, ws, s)
                               : launch_gemv_q6s(w, X, out, nvec, rows, cols, row_bytes, ws, s, cnt);
       }

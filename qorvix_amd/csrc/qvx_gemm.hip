@@ -1489,6 +1489,14 @@ bool stream_key(hipStream_t s, int& dev, unsigned long long& sid) {
 
 }  // namespace
 
+// Whether `s` is recording a graph (an unanswered query counts as recording).
+bool stream_capturing(hipStream_t s) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &cs) == hipSuccess) return cs != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
+
 // Stream-ordered temporary from the library's pool (nullptr on failure) and its release.
 void* gemm_temp_alloc(size_t bytes, hipStream_t s) {
   hipMemPool_t pool = device_pool();

@@ -399,10 +399,15 @@ __device__ inline const float* task_x(const float* X, int cols, int S, int t) {
   return X + (size_t)v * cols + L::xoff(s, part >> 1) + 8 * (part & 1);
 }
 
+// The fixed-point form of a task's 8 elements: signed bytes of qh and ql in element order, the sum of q
+// over the task's run of 16, and the slot's step sx.  The 2R lanes of a slot agree on its largest |x|.
+struct Quant8 {
+  uint32_t h[2], l[2];
+  int sum;
+  float sx;
+};
 template <int R>
-__device__ inline void convert_task(const float4 x0, const float4 x1, int t, bool store, uint32_t* xs,
-                                    float* sx_out = nullptr) {
-  const int vs = t / (2 * R), part = t % (2 * R), run = part >> 1, hf = part & 1;
+__device__ inline void convert_quant(const float4 x0, const float4 x1, Quant8& q) {
   float a = fmaxf(fmaxf(fmaxf(fabsf(x0.x), fabsf(x0.y)), fmaxf(fabsf(x0.z), fabsf(x0.w))),
                   fmaxf(fmaxf(fabsf(x1.x), fabsf(x1.y)), fmaxf(fabsf(x1.z), fabsf(x1.w))));
   // 0 when the eight elements are finite, NaN otherwise (x * 0 is NaN for +-Inf and NaN)
@@ -434,16 +439,30 @@ __device__ inline void convert_task(const float4 x0, const float4 x1, int t, boo
 #pragma unroll
   for (int i = 0; i < 4; ++i) sq = __builtin_amdgcn_sdot2(__builtin_bit_cast(short2_t, p[i]), ones, sq, false);
   sq += dpp<kXor1>(sq);  // the other half of the run
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    q.h[i] = __builtin_amdgcn_perm(hs[2 * i + 1], hs[2 * i], 0x06040200u);  // low bytes of the four 16-bit lanes
+    q.l[i] = __builtin_amdgcn_perm(ls[2 * i + 1], ls[2 * i], 0x06040200u);
+  }
+  q.sum = sq;
+  q.sx = a * (1.0f / 16383.0f) + z;
+}
+template <int R>
+__device__ inline void convert_task(const float4 x0, const float4 x1, int t, bool store, uint32_t* xs,
+                                    float* sx_out = nullptr) {
+  const int vs = t / (2 * R), part = t % (2 * R), run = part >> 1, hf = part & 1;
+  Quant8 q;
+  convert_quant<R>(x0, x1, q);
   if (store) {
     uint32_t* o = xs + (size_t)vs * xq_words<R>();
     const int w = 4 * run + 2 * hf;
-    o[w] = __builtin_amdgcn_perm(hs[1], hs[0], 0x06040200u);  // low bytes of the four 16-bit lanes
-    o[w + 1] = __builtin_amdgcn_perm(hs[3], hs[2], 0x06040200u);
-    o[4 * R + w] = __builtin_amdgcn_perm(ls[1], ls[0], 0x06040200u);
-    o[4 * R + w + 1] = __builtin_amdgcn_perm(ls[3], ls[2], 0x06040200u);
-    if (hf == 0) o[8 * R + run] = (uint32_t)sq;
-    if (part == 0) o[9 * R] = __builtin_bit_cast(uint32_t, a * (1.0f / 16383.0f) + z);
-    if (part == 0 && sx_out) *sx_out = a * (1.0f / 16383.0f) + z;
+    o[w] = q.h[0];
+    o[w + 1] = q.h[1];
+    o[4 * R + w] = q.l[0];
+    o[4 * R + w + 1] = q.l[1];
+    if (hf == 0) o[8 * R + run] = (uint32_t)q.sum;
+    if (part == 0) o[9 * R] = __builtin_bit_cast(uint32_t, q.sx);
+    if (part == 0 && sx_out) *sx_out = q.sx;
   }
 }
 

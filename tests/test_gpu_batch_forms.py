@@ -1,0 +1,106 @@
+"""The batched form that reads Q8_0 / Q4_0 / Q5_0 weights once for many vectors on the matrix cores
+(k_gemv_int): bit-identical to single vectors, and within the GEMV bar of the fp64 oracle."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import oracle
+import qorvix_amd as qvx
+from conftest import max_rel
+from test_gpu_kernels import dev, f32bits, random_weight
+
+pytestmark = pytest.mark.gpu
+
+GEMV_TOL = 1e-3
+
+
+def _run(torch, w, t, X, rows, cols, bias=None):
+    n = X.shape[0]
+    out = torch.full((n, rows), float("nan"), dtype=torch.float32, device="cuda")
+    st = torch.cuda.current_stream().cuda_stream
+    rc = qvx.qmatmul_n_bias(out.data_ptr(), w.data_ptr(), t, X.data_ptr(), bias.data_ptr() if bias is not None else 0,
+                            n, rows, cols, st)
+    assert rc == qvx.OK, qvx.strerror(rc)
+    return out
+
+
+def _singles(torch, w, t, X, rows, cols, which):
+    return torch.cat([_run(torch, w, t, X[i:i + 1].contiguous(), rows, cols) for i in which])
+
+
+def _check(torch, t, rows, cols, n, seed, bias=False, zero_vec=False, tol=GEMV_TOL, offset=0):
+    rng = np.random.default_rng(seed)
+    w_np = random_weight(t, rows, cols, rng)
+    X_np = rng.standard_normal((n, cols)).astype(np.float32)
+    if zero_vec:
+        X_np[1] = 0.0
+    w, X = dev(torch, np.concatenate([np.zeros(offset, np.uint8), w_np]))[offset:], dev(torch, X_np)
+    got = _run(torch, w, t, X, rows, cols)
+    which = sorted({0, min(1, n - 1), n // 2, max(n - 2, 0), n - 1})
+    one = _singles(torch, w, t, X, rows, cols, which)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(f32bits(got[which].cpu().numpy()), f32bits(one.cpu().numpy()))
+    ref = oracle.matmul_f64(w_np, t, X_np[which], len(which), rows, cols)
+    assert max_rel(got[which].cpu().numpy(), ref) <= tol
+    if bias:
+        b = dev(torch, rng.standard_normal(rows).astype(np.float32))
+        gb = _run(torch, w, t, X, rows, cols, b)
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(f32bits(gb.cpu().numpy()), f32bits((got + b).cpu().numpy()))
+
+
+# Slots of 64 elements: one slot; a short row's padded tree (6 of 8, 20 of 32); exactly one 64-slot block;
+# one slot past it; several blocks with a partial last one.  Rows: one, ragged, whole tiles.  Vectors: the
+# fewest (9, or 5 on large weights), one tile, one past it, several workgroups; few waves take the K parts,
+# many do not.
+INT_CASES = [(1, 64, 9), (4, 512, 12), (36, 2560, 16), (4200, 4096, 5), (8200, 4096, 7), (1, 64, 17), (33, 384, 20), (40, 1280, 33), (64, 4096, 17), (70, 4096, 65), (31, 4160, 18),
+             (100, 11008, 24), (1030, 4096, 70), (2080, 1024, 130), (1100, 4096, 260)]
+
+
+@pytest.mark.parametrize("t", [qvx.Q8_0, qvx.Q4_0, qvx.Q5_0])
+@pytest.mark.parametrize("rows,cols,n", INT_CASES)
+def test_int_batches_match_single_vectors(cuda, t, rows, cols, n):
+    _check(cuda, t, rows, cols, n, seed=rows + cols + n, bias=True, zero_vec=True)
+
+
+def test_int_batch_keeps_non_finite_vectors_apart(cuda):
+    """A non-finite activation makes its own vector's outputs NaN and leaves the tile's other vectors as they
+    are."""
+    rng = np.random.default_rng(3)
+    t, rows, cols, n = qvx.Q8_0, 50, 512, 19
+    w_np = random_weight(t, rows, cols, rng)
+    X_np = rng.standard_normal((n, cols)).astype(np.float32)
+    w = dev(cuda, w_np)
+    clean = _run(cuda, w, t, dev(cuda, X_np), rows, cols).cpu().numpy()
+    X_np[3, 7], X_np[16, 500] = np.inf, np.nan
+    got = _run(cuda, w, t, dev(cuda, X_np), rows, cols).cpu().numpy()
+    assert np.isnan(got[[3, 16]]).all()
+    keep = [i for i in range(n) if i not in (3, 16)]
+    np.testing.assert_array_equal(f32bits(got[keep]), f32bits(clean[keep]))
+
+
+def test_int_batch_in_plan_and_capture(cuda):
+    """A plan's batch (its workspace made at instantiation) and a captured call (no temporary) give the eager
+    call's bits on every replay."""
+    from qorvix_amd import decode
+    rng = np.random.default_rng(11)
+    t, rows, cols, n = qvx.Q4_0, 96, 1024, 21
+    w = decode.DevWeight(dev(cuda, random_weight(t, rows, cols, rng)), t, rows, cols)
+    X = dev(cuda, rng.standard_normal((n, cols)).astype(np.float32))
+    want = f32bits(qvx.qmatmul_t(w.data, t, X, rows, cols).cpu().numpy())
+    out = cuda.empty((n, rows), dtype=cuda.float32, device="cuda")
+    plan = decode.Plan()
+    plan.add(out, w, X, n)
+    plan.instantiate()
+    cap = cuda.empty((n, rows), dtype=cuda.float32, device="cuda")
+    graph = cuda.cuda.CUDAGraph()
+    with cuda.cuda.graph(graph):
+        qvx.qmatmul_t(w.data, t, X, rows, cols, out=cap)
+    for _ in range(3):
+        out.zero_(), cap.zero_()
+        plan.launch(cuda.cuda.current_stream().cuda_stream)
+        graph.replay()
+        cuda.cuda.synchronize()
+        np.testing.assert_array_equal(f32bits(out.cpu().numpy()), want)
+        np.testing.assert_array_equal(f32bits(cap.cpu().numpy()), want)
