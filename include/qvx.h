@@ -71,7 +71,8 @@ const char* qvx_strerror(int code);
 /* 1 if qvx_qmatmul / qvx_qmatmul_n compute `type` (qmatmul.cpp:24-26, qmatmulSupports): every
  * type the reference dequantises (F32, F16, BF16, Q8_0, Q8_1, Q4_0, Q4_1, Q5_0, Q5_1, Q4_K, Q5_K,
  * Q6_K).  Q8_0 / Q4_0 / Q5_0 / Q4_K / Q5_K / Q6_K run on the integer fast kernels, F32 / F16 /
- * BF16 on the float kernel, Q8_1 / Q4_1 / Q5_1 and unaligned weights on a generic kernel.
+ * BF16 on the fp32-activation kernels, and so do Q8_1 / Q4_1 / Q5_1, unaligned weights and row pitches
+ * that are not multiples of 16 bytes.
  * qvx_qgemm_f16 computes the same types. */
 int qvx_supports(uint32_t type);
 
@@ -125,7 +126,9 @@ int qvx_qmatmul(float* d_out, const void* d_w, uint32_t type, const float* d_x, 
  * and 5-bit formats), on the one-vector kernel's shapes, run on a matrix-core form that converts the
  * activations once into a stream-ordered temporary (n_vec * cols * 2.06 bytes, at most about 64 MiB: larger
  * batches run in parts) or a plan's workspace, and reads the weights once per 16 to 64 vectors; on a
- * capturing stream they keep the one-vector kernel's launches, which take no temporary. */
+ * capturing stream they keep the one-vector kernel's launches, which take no temporary.
+ * The fp32-activation kernels (see qvx_supports) read the weights once per 8 vectors from 9 vectors (from 5
+ * on 8192 rows or more), per 4 below. */
 int qvx_qmatmul_n(float* d_out, const void* d_w, uint32_t type, const float* d_X, int n_vec,
                   int rows, int cols, void* stream);
 

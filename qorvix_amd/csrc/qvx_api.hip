@@ -31,8 +31,11 @@ void launch_swiglu(float* out, const float* g, const float* u, size_t n, hipStre
 void launch_swiglu_interleaved(float* out, const float* y, int nvec, int ffn, hipStream_t s);
 void* gemm_temp_alloc(size_t bytes, hipStream_t s);
 void gemm_temp_free(void* p, hipStream_t s);
-bool launch_gemv_float(uint32_t t, const void* w, const float* X, float* Y, int nvec, int rows, int cols,
-                       size_t row_bytes, hipStream_t s);
+bool gemv_float_tiled(int nvec, int rows);
+bool launch_gemv_float(uint32_t t, const void* w, const float* X, float* Y, const float* bias, int nvec, int rows,
+                       int cols, size_t row_bytes, hipStream_t s);
+bool launch_gemv_loose(uint32_t t, const void* w, const float* X, float* Y, const float* bias, int nvec, int rows,
+                       int cols, size_t row_bytes, hipStream_t s);
 int gemv_mx_max_nv(int cols);
 int gemv_mxj_supported(int cols);
 bool launch_gemv_mxj_q4k(const void* w, const float* X, float* Y, int nvec, int rows, int cols, size_t row_bytes,
@@ -153,6 +156,18 @@ inline int check_matmul(uint32_t type, int cols, const TypeInfo** ti) {
 }
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
+
+// Whether a call runs on the fp32-activation kernels' tiled form, which adds the bias itself: a large
+// enough batch of unquantised weights in whole chunks, or of block weights that no integer kernel
+// takes (unaligned ones, and Q4_1 / Q5_1 / Q8_1).
+inline bool float_tiled(uint32_t type, int nvec, int rows, int cols, bool fast, const void* X) {
+  if (!gemv_float_tiled(nvec, rows) || !aligned16(X)) return false;
+  switch (type) {
+    case T_F32: case T_F16: case T_BF16: return fast && cols % (type == T_F32 ? 4 : 8) == 0 && cols <= 32768;
+    case T_Q4_1: case T_Q5_1: case T_Q8_1: return true;
+    default: return !fast;
+  }
+}
 
 // Whether a Q4_K batch takes the many-vector form rather than chunks of 8 vectors.  The form costs
 // a conversion launch and a K-range chain per wave whatever the batch (17-22 us in graph replays on
@@ -333,7 +348,7 @@ int gemv(float* out, const void* w, uint32_t type, const float* X, int nvec, int
       return hip_status();
     }
   }
-  if (epi.bias) {  // every other route: the plain product, then the bias add
+  if (epi.bias && !float_tiled(type, nvec, rows, cols, fast, X)) {  // every other route: the plain product, then the bias add
     GemvEpi plain = epi;
     plain.bias = nullptr;
     if (int rc = gemv(out, w, type, X, nvec, rows, cols, s, plain); rc != QVX_OK) return rc;
@@ -342,12 +357,12 @@ int gemv(float* out, const void* w, uint32_t type, const float* X, int nvec, int
   }
   // Unquantised weights stream through the float kernel.
   if (fast && (type == T_F32 || type == T_F16 || type == T_BF16) &&
-      launch_gemv_float(type, w, X, out, nvec, rows, cols, row_bytes, s))
+      launch_gemv_float(type, w, X, out, epi.bias, nvec, rows, cols, row_bytes, s))
     return hip_status();
   // The fast kernels take any number of vectors, a few per launch; each vector's arithmetic is the
   // same in every launch, so batches stay bit-identical to single vectors.  Q4_K runs on the matrix
   // cores (up to gemv_mx_max_nv vectors per launch), the other formats on the VALU kernel; shapes
-  // neither covers go to the generic kernel.
+  // neither covers go to the fp32-activation kernels (qvx_gemv_f.hip).
   // Q4_K batches of two or more vectors, 8 at a time: a chunk of up to 3 vectors (2 on long rows)
   // runs on the one-vector kernel, several vectors a launch (measured faster there); larger chunks
   // take a batched matrix-core form: the one that stages a whole row's activation fragments in LDS
@@ -387,6 +402,8 @@ int gemv(float* out, const void* w, uint32_t type, const float* X, int nvec, int
   }
   if (fast && launch_gemv_fast(type, w, X, out, nvec, rows, cols, row_bytes, epi, s)) return hip_status();
   if (epi.flags()) return refused();  // fused_route() promised a fused kernel
+  if (launch_gemv_loose(type, w, X, out, epi.bias, nvec, rows, cols, row_bytes, s)) return hip_status();
+  if (epi.bias) return refused();  // float_tiled() promised the loose form
   for (int v0 = 0; v0 < nvec; v0 += 16) {
     const int nv = nvec - v0 < 16 ? nvec - v0 : 16;
     if (!launch_gemv_generic(type, w, X + (size_t)v0 * cols, out + (size_t)v0 * rows, rows, cols, nv, row_bytes, s))

@@ -58,7 +58,7 @@ inline bool can_dequantize(uint32_t t) {
 // Types the GEMV / GEMM kernels compute.
 // Every type the reference's qmatmul accepts (qmatmulSupports = canDequantize && traits,
 // runtime/src/qmatmul.cpp:24-26): Q8_0 / Q4_0 / Q4_K / Q6_K on the fast kernels, the others on the
-// generic kernel.
+// fp32-activation kernels.
 inline bool gemv_supports(uint32_t t) { return can_dequantize(t); }
 
 // Block geometry of the four GEMV formats.  A "panel" is PB consecutive blocks of a row: 2048

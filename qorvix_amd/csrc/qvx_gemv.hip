@@ -37,7 +37,7 @@
 //    (runtime/include/qorvix/runtime/qmatmul.hpp:31-32).
 //
 // Requirements checked by the launcher: W and X 16-byte aligned, row pitch a multiple of 16 bytes,
-// K a whole number of slots, S' <= 1024.  Other shapes go to the generic kernel in qvx_dequant.hip.
+// K a whole number of slots, S' <= 1024.  Other shapes go to the fp32-activation kernels in qvx_gemv_f.hip.
 #include "qvx_gemv_valu.hpp"
 
 namespace qvx {
@@ -676,7 +676,7 @@ bool gemv_fast_fusable(uint32_t t, int cols, size_t row_bytes, const GemvEpi& ep
 }
 
 // Fast-path GEMV for nvec >= 1 on 16-byte-aligned rows of Q8_0 / Q4_0 / Q5_0 / Q4_K / Q5_K / Q6_K.  Returns
-// false, having launched nothing, when the shape needs the generic kernel.
+// false, having launched nothing, when the shape needs the fp32-activation kernels.
 bool launch_gemv_fast(uint32_t t, const void* w, const float* X, float* Y, int nvec, int rows, int cols,
                       size_t row_bytes, const GemvEpi& epi, hipStream_t s) {
   switch (t) {

@@ -683,7 +683,7 @@ constexpr int max_rows() {
 
 // Slot geometry of a row: S slots, padded group width Sp, groups per workgroup G.  Returns false
 // when K is not a whole number of slots, a row has more than 1024 slots, or two vectors'
-// converted activations do not fit in LDS: the generic kernel takes those.
+// converted activations do not fit in LDS: the fp32-activation kernels take those.
 template <uint32_t T>
 inline bool geometry(int cols, size_t row_bytes, Geo& geo) {
   constexpr int E = Lane<T>::kSlotElems;

@@ -1,5 +1,7 @@
-"""The batched form that reads Q8_0 / Q4_0 / Q5_0 weights once for many vectors on the matrix cores
-(k_gemv_int): bit-identical to single vectors, and within the GEMV bar of the fp64 oracle."""
+"""The batched forms that read the weights once for many vectors: Q8_0 / Q4_0 / Q5_0 on the matrix cores
+(k_gemv_int), and the fp32-activation kernels (k_gemv_float, k_gemv_float_many): unquantised weights, and block
+formats at alignments and row pitches the integer kernels do not take.  Batches are bit-identical to single
+vectors, and within the GEMV bar of the fp64 oracle."""
 from __future__ import annotations
 
 import numpy as np
@@ -13,6 +15,10 @@ from test_gpu_kernels import dev, f32bits, random_weight
 pytestmark = pytest.mark.gpu
 
 GEMV_TOL = 1e-3
+# fp32 activations and exact weight values: an output is a chain of 8 FMAs, 6 tree adds and K / 512 segment
+# adds, so its error is at most (14 + K / 512) 2^-24 sum |w x|; with sum |w x| <= 0.4 sqrt(K) max |ref| for
+# these inputs and K <= 11008, 36 * 6e-8 * 42.
+FP32_TOL = 9e-5
 
 
 def _run(torch, w, t, X, rows, cols, bias=None):
@@ -78,6 +84,51 @@ def test_int_batch_keeps_non_finite_vectors_apart(cuda):
     assert np.isnan(got[[3, 16]]).all()
     keep = [i for i in range(n) if i not in (3, 16)]
     np.testing.assert_array_equal(f32bits(got[keep]), f32bits(clean[keep]))
+
+
+# Chunks of 16 bytes: less than a stage of 8, a partial stage, a partial segment of 64, one segment, one
+# chunk past it; tiles of 32 and (from 256 workgroups) of 64.
+FLOAT_CASES = [(1, 8, 9), (33, 40, 9), (17, 384, 20), (48, 512, 33), (65, 520, 64), (40, 1536, 31), (1040, 384, 1030)]
+
+
+@pytest.mark.parametrize("t", [qvx.F16, qvx.BF16, qvx.F32])
+@pytest.mark.parametrize("rows,cols,n", FLOAT_CASES)
+def test_float_batches_match_single_vectors(cuda, t, rows, cols, n):
+    _check(cuda, t, rows, cols, n, seed=rows + cols + n, bias=True, zero_vec=True)
+
+
+# Block formats on the fp32-activation kernels: the types no integer kernel computes, row pitches that are
+# not multiples of 16 bytes (Q6_K rows of an odd number of super-blocks lie at 2-byte offsets), and weights
+# whose first byte is unaligned.  K: less than a segment of 512, a partial last one, many.
+LOOSE_CASES = [(qvx.Q6_K, 1, 256, 0), (qvx.Q6_K, 37, 768, 0), (qvx.Q6_K, 300, 5632, 0), (qvx.Q6_K, 70, 11008, 0),
+               (qvx.Q6_K, 33, 2048, 2), (qvx.Q8_0, 45, 96, 0), (qvx.Q8_0, 130, 4128, 0), (qvx.Q4_0, 45, 192, 0),
+               (qvx.Q5_0, 77, 832, 0), (qvx.Q4_1, 50, 1056, 0), (qvx.Q5_1, 50, 544, 0), (qvx.Q8_1, 50, 4096, 0),
+               (qvx.Q4_K, 40, 1280, 1), (qvx.Q5_K, 40, 1280, 4), (qvx.F16, 40, 520, 2), (qvx.BF16, 40, 520, 2),
+               (qvx.F32, 40, 520, 4)]
+
+
+@pytest.mark.parametrize("t,rows,cols,offset", LOOSE_CASES)
+@pytest.mark.parametrize("n", [1, 3, 9, 70])
+def test_loose_blocks(cuda, t, rows, cols, offset, n):
+    _check(cuda, t, rows, cols, n, seed=rows + cols + n, bias=True, tol=FP32_TOL, offset=offset)
+
+
+def test_loose_rows_past_the_staging_budget(cuda):
+    """Rows of more than 32768 elements read their activations from global memory, four vectors a launch."""
+    _check(cuda, qvx.Q4_1, 5, 33024, 7, seed=5, tol=2e-4)
+
+
+def test_unaligned_row_pitch_rmsnorm(cuda):
+    """A fused norm on rows no kernel folds it into: the bits of the standalone norm followed by the product."""
+    t, rows, cols = qvx.Q6_K, 40, 1536
+    rng = np.random.default_rng(cols)
+    w = dev(cuda, random_weight(t, rows, cols, rng))
+    X = dev(cuda, rng.standard_normal((3, cols)).astype(np.float32))
+    nw = dev(cuda, (1 + 0.1 * rng.standard_normal(cols)).astype(np.float32))
+    got = qvx.qmatmul_rmsnorm_t(w, t, X, nw, 1e-5, rows, cols)
+    want = qvx.qmatmul_t(w, t, qvx.rmsnorm_t(X, nw, 1e-5), rows, cols)
+    cuda.cuda.synchronize()
+    np.testing.assert_array_equal(f32bits(got.cpu().numpy()), f32bits(want.cpu().numpy()))
 
 
 def test_int_batch_in_plan_and_capture(cuda):
