@@ -35,15 +35,15 @@ __device__ inline V ldu(const uint8_t* p) {
 }
 
 // ---- weight chunks -----------------------------------------------------------------------------------
-// Src<T>: E elements a chunk; kU chunks a lane of the streaming form requests at a time; Raw = a chunk's bytes in registers; load() issues its loads (chunk c of the
-// row at rp); widen() forms the fp32 values.
+// Src<T>: E elements a chunk; kU chunks a lane of the streaming form requests at a time; kSeg bytes a segment of
+// 64 chunks; Raw = a chunk's bytes in registers; load() issues its loads (chunk l of the segment at p: the
+// lane's part of the address is the same in every segment); widen() forms the fp32 values.
 template <uint32_t T> struct Src;
 
 template <uint32_t T> struct SrcPlain {  // 16 bytes of fp32 / fp16 / bf16 values
-  static constexpr int E = T == T_F32 ? 4 : 8, kU = 8;
+  static constexpr int E = T == T_F32 ? 4 : 8, kU = 8, kSeg = 1024;
   typedef uint4 Raw;
-  static __device__ inline Raw none() { return make_uint4(0, 0, 0, 0); }
-  static __device__ inline Raw load(const uint8_t* rp, int c) { return *reinterpret_cast<const uint4*>(rp + (size_t)16 * c); }
+  static __device__ inline Raw load(const uint8_t* p, int l) { return *reinterpret_cast<const uint4*>(p + 16 * l); }
   static __device__ inline void widen(const Raw& w, float (&f)[E]) {
     const uint32_t d[4] = {w.x, w.y, w.z, w.w};
 #pragma unroll
@@ -67,11 +67,10 @@ template <> struct Src<T_BF16> : SrcPlain<T_BF16> {};
 // Unquantised weights at any alignment: 8 elements a chunk.
 template <uint32_t T> struct SrcLoose;
 template <> struct SrcLoose<T_F32> {
-  static constexpr int E = 8, kU = 4;
+  static constexpr int E = 8, kU = 4, kSeg = 2048;
   struct Raw { uint4 a, b; };
-  static __device__ inline Raw none() { return {}; }
-  static __device__ inline Raw load(const uint8_t* rp, int c) {
-    return {ldu<uint4>(rp + (size_t)32 * c), ldu<uint4>(rp + (size_t)32 * c + 16)};
+  static __device__ inline Raw load(const uint8_t* p, int l) {
+    return {ldu<uint4>(p + 32 * l), ldu<uint4>(p + 32 * l + 16)};
   }
   static __device__ inline void widen(const Raw& w, float (&f)[8]) {
     const uint32_t d[8] = {w.a.x, w.a.y, w.a.z, w.a.w, w.b.x, w.b.y, w.b.z, w.b.w};
@@ -80,10 +79,10 @@ template <> struct SrcLoose<T_F32> {
   }
 };
 template <> struct SrcLoose<T_F16> : SrcPlain<T_F16> {
-  static __device__ inline Raw load(const uint8_t* rp, int c) { return ldu<uint4>(rp + (size_t)16 * c); }
+  static __device__ inline Raw load(const uint8_t* p, int l) { return ldu<uint4>(p + 16 * l); }
 };
 template <> struct SrcLoose<T_BF16> : SrcPlain<T_BF16> {
-  static __device__ inline Raw load(const uint8_t* rp, int c) { return ldu<uint4>(rp + (size_t)16 * c); }
+  static __device__ inline Raw load(const uint8_t* p, int l) { return ldu<uint4>(p + 16 * l); }
 };
 
 // The formats of 32-element blocks: codes q at byte kQ (8 bits: element e at kQ + e; 4 bits: low nibbles
@@ -91,12 +90,11 @@ template <> struct SrcLoose<T_BF16> : SrcPlain<T_BF16> {
 // (kM) or a constant kOff subtracted from the code.
 template <int BB, int kQ, bool kByte, int kH, bool kM, int kOff>
 struct Src32 {
-  static constexpr int E = 8, kU = 4;
+  static constexpr int E = 8, kU = 4, kSeg = 16 * BB;
   struct Raw { uint2 q; uint32_t h, dm; };
-  static __device__ inline Raw none() { return {}; }
-  static __device__ inline Raw load(const uint8_t* rp, int c) {
-    const uint8_t* b = rp + (size_t)(c >> 2) * BB;
-    const int e0 = 8 * (c & 3);
+  static __device__ inline Raw load(const uint8_t* p, int l) {
+    const uint8_t* b = p + (l >> 2) * BB;
+    const int e0 = 8 * (l & 3);
     Raw r;
     r.q = ldu<uint2>(b + kQ + (kByte ? e0 : (e0 & 15)));
     if (!kByte) r.q.x >>= e0 < 16 ? 0 : 4, r.q.y >>= e0 < 16 ? 0 : 4;
@@ -106,13 +104,13 @@ struct Src32 {
     return r;
   }
   static __device__ inline void widen(const Raw& r, float (&f)[8]) {
-    const float d = f16lo(r.dm), m = kM ? f16hi(r.dm) : 0.0f;
+    const float d = f16lo(r.dm), m = kM ? f16hi(r.dm) : -(float)kOff * d;
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
       const uint32_t w = k < 4 ? r.q.x >> (8 * k) : r.q.y >> (8 * k - 32);
       int q = kByte ? (int)(int8_t)w : (int)(w & 15u);
       if constexpr (kH >= 0) q |= (int)(((r.h >> k) & 1u) << 4);
-      f[k] = kM ? __builtin_fmaf((float)q, d, m) : (float)(q - kOff) * d;
+      f[k] = __builtin_fmaf((float)q, d, m);  // the product is exact: one rounding at most
     }
   }
 };
@@ -126,11 +124,10 @@ template <> struct Src<T_Q5_1> : Src32<24, 8, false, 4, true, 0> {};
 // Q4_K / Q5_K: d, dmin and the 12 bytes of 6-bit scales and mins, Q5_K's fifth bits, the nibbles.
 template <bool kFive>
 struct SrcK45 {
-  static constexpr int E = 8, kU = 4, BB = kFive ? 176 : 144;
+  static constexpr int E = 8, kU = 4, BB = kFive ? 176 : 144, kSeg = 2 * BB;
   struct Raw { uint4 hd; uint2 q, h; uint32_t j; };
-  static __device__ inline Raw none() { return {}; }
-  static __device__ inline Raw load(const uint8_t* rp, int c) {
-    const uint8_t* b = rp + (size_t)(c >> 5) * BB;
+  static __device__ inline Raw load(const uint8_t* p, int c) {
+    const uint8_t* b = p + (c >> 5) * BB;
     const int e0 = 8 * (c & 31), g = e0 >> 6, l = e0 & 31, hi = (e0 >> 5) & 1;
     Raw r;
     r.hd = ldu<uint4>(b);
@@ -159,11 +156,10 @@ template <> struct Src<T_Q4_K> : SrcK45<false> {};
 template <> struct Src<T_Q5_K> : SrcK45<true> {};
 
 template <> struct Src<T_Q6_K> {
-  static constexpr int E = 8, kU = 4;
+  static constexpr int E = 8, kU = 4, kSeg = 420;
   struct Raw { uint2 l, h; uint32_t sc, d; };
-  static __device__ inline Raw none() { return {}; }
-  static __device__ inline Raw load(const uint8_t* rp, int c) {
-    const uint8_t* b = rp + (size_t)(c >> 5) * 210;
+  static __device__ inline Raw load(const uint8_t* p, int c) {
+    const uint8_t* b = p + (c >> 5) * 210;
     const int e0 = 8 * (c & 31), h = e0 >> 7, quarter = (e0 >> 5) & 3, l = e0 & 31;
     Raw r;
     r.l = ldu<uint2>(b + 64 * h + 32 * (quarter & 1) + l);
@@ -176,11 +172,12 @@ template <> struct Src<T_Q6_K> {
     return r;
   }
   static __device__ inline void widen(const Raw& r, float (&f)[8]) {
-    const float ds = f16lo(r.d) * (float)(int)(int8_t)r.sc;
+    const float ds = f16lo(r.d) * (float)(int)(int8_t)r.sc, m = -32.0f * ds;
     const uint32_t q[2] = {(r.l.x & 0x0F0F0F0Fu) | ((r.h.x & 0x03030303u) << 4),
                            (r.l.y & 0x0F0F0F0Fu) | ((r.h.y & 0x03030303u) << 4)};
 #pragma unroll
-    for (int k = 0; k < 8; ++k) f[k] = ds * ((float)((q[k >> 2] >> (8 * (k & 3))) & 0xFFu) - 32.0f);
+    for (int k = 0; k < 8; ++k)  // ds (q - 32), rounded once
+      f[k] = __builtin_fmaf((float)((q[k >> 2] >> (8 * (k & 3))) & 0xFFu), ds, m);
   }
 };
 
@@ -233,13 +230,18 @@ __global__ __launch_bounds__(1024) void k_gemv_float(const uint8_t* __restrict__
   // 96 -> 47 us); unquantised chunks, eight 16-byte loads a block already, do without (4096 x 4096 fp16:
   // 9.3 us with, 8.7 without).
   constexpr bool kAhead = S::kU < 8;
-  int r = (int)blockIdx.x * nw + wave, c0 = lane;
+  // Lanes past the row's last chunk repeat it (their sums skip it), so no load is in a branch.
+  const int nseg = (nchunk + 63) / 64, lastc = min(lane, nchunk - 64 * (nseg - 1) - 1);
+  int r = (int)blockIdx.x * nw + wave, g0 = 0;
   auto request = [&](typename S::Raw (&w)[kU]) __attribute__((always_inline)) {
     const uint8_t* rp = W + (size_t)min(r, rows - 1) * row_bytes;
 #pragma unroll
-    for (int u = 0; u < kU; ++u) w[u] = r < rows && c0 + 64 * u < nchunk ? S::load(rp, c0 + 64 * u) : S::none();
-    c0 += 64 * kU;
-    if (c0 - lane >= nchunk) c0 = lane, r += stride;
+    for (int u = 0; u < kU; ++u) {
+      const int g = min(g0 + u, nseg - 1);
+      w[u] = S::load(rp + (size_t)g * S::kSeg, g == nseg - 1 ? lastc : lane);
+    }
+    g0 += kU;
+    if (g0 >= nseg) g0 = 0, r += stride;
   };
   typename S::Raw w[kU], wn[kU];
   request(w);
@@ -306,8 +308,8 @@ __global__ __launch_bounds__(1024) void k_gemv_float(const uint8_t* __restrict__
 // sums 8 (q % 2) + 16 (q / 2) + j), DPP adds the rest -- the butterfly's own pairs.
 // Bound by the FMAs; the LDS reads that feed them take half their time.  Measured on MI355X, graph-replayed:
 // fp16 384 x 1536 at 256 vectors 12.6 us, where 64 launches of the streaming form took 290; 14336 x 4096 at
-// 16 vectors 110 -> 58 us; Q6_K 32000 x 3072 at 16 570 -> 170 us (the byte-by-byte decode this file's block
-// chunks replaced; its one-vector call 126 -> 47, 2048 x 5632 24 -> 11.6).
+// 16 vectors 110 -> 57 us; Q6_K 32000 x 3072 at 16 570 -> 114 us (the byte-by-byte decode this file's block
+// chunks replaced; its one-vector call 126 -> 43, 2048 x 5632 24 -> 7.8).
 constexpr int kTV = 8, kTR = 4, kTS = 2, kTW = 8;  // vectors, rows a wave, segments a stage, waves
 template <typename S>
 __global__ __launch_bounds__(64 * kTW) void k_gemv_float_many(const uint8_t* __restrict__ W, const float* __restrict__ X,
@@ -320,6 +322,7 @@ __global__ __launch_bounds__(64 * kTW) void k_gemv_float_many(const uint8_t* __r
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r0 = ((int)blockIdx.x * kTW + wave) * kTR, v0 = (int)blockIdx.y * kTV;
   const int nchunk = cols / E, nst = (nchunk + 64 * kTS - 1) / (64 * kTS);
+  const int nseg = (nchunk + 63) / 64, lastc = min(lane, nchunk - 64 * (nseg - 1) - 1);  // as the streaming form's
 
   auto load_x = [&](int st, float4 (&x)[NX]) __attribute__((always_inline)) {
 #pragma unroll
@@ -341,8 +344,9 @@ __global__ __launch_bounds__(64 * kTW) void k_gemv_float_many(const uint8_t* __r
     for (int u = 0; u < kTS; ++u)
 #pragma unroll
       for (int i = 0; i < kTR; ++i) {
-        const int c = 64 * (kTS * st + u) + lane;
-        w[u][i] = c < nchunk ? S::load(W + (size_t)min(r0 + i, rows - 1) * row_bytes, c) : S::none();
+        const int g = min(kTS * st + u, nseg - 1);
+        w[u][i] = S::load(W + (size_t)min(r0 + i, rows - 1) * row_bytes + (size_t)g * S::kSeg,
+                          g == nseg - 1 ? lastc : lane);
       }
   };
 
@@ -364,10 +368,11 @@ __global__ __launch_bounds__(64 * kTW) void k_gemv_float_many(const uint8_t* __r
 #pragma unroll
       for (int i = 0; i < kTR; ++i) S::widen(w[u][i], f[i]);
       const int c = 64 * (kTS * st + u) + lane;
-      if (more)  // this segment's registers take the next stage's
+      const int gn = min(kTS * (st + 1) + u, nseg - 1);  // this segment's registers take the next stage's
 #pragma unroll
-        for (int i = 0; i < kTR; ++i)
-          w[u][i] = c + 64 * kTS < nchunk ? S::load(W + (size_t)min(r0 + i, rows - 1) * row_bytes, c + 64 * kTS) : S::none();
+      for (int i = 0; i < kTR; ++i)
+        w[u][i] = S::load(W + (size_t)min(r0 + i, rows - 1) * row_bytes + (size_t)gn * S::kSeg,
+                          gn == nseg - 1 ? lastc : lane);
       if (c < nchunk) {
 #pragma unroll
         for (int v = 0; v < kTV; ++v) {
