@@ -170,7 +170,8 @@ int qvx_swiglu(float* d_out, const float* d_gate, const float* d_up, size_t n, v
  * (d_out[i] is bit-identical to that call on member i alone); a member with rows[i] <= 0 computes
  * nothing.  Up to 4 Q4_K members and one Q6_K member with aligned operands and cols a multiple of
  * 256 up to 16384 (of 512 with a norm) run as ONE launch (the dispatch ramp and drain paid once,
- * the norm folded into each workgroup's activation conversion); other groups run member by member. */
+ * the norm folded into each workgroup's activation conversion), and so do 2 to 4 members of one Q8_0 /
+ * Q4_0 / Q5_0 / Q5_K / Q6_K type without a norm; other groups run member by member. */
 #define QVX_GROUP_MAX 8
 int qvx_qmatmul_group(float* const* d_out, const void* const* d_w, const uint32_t* types, const int* rows, int n,
                       const float* d_x, const float* d_norm_w, float eps, int cols, void* stream);
@@ -323,7 +324,9 @@ int qvx_plan_join(qvx_plan* plan);
 /* Number of recorded calls. */
 int qvx_plan_size(const qvx_plan* plan);
 /* Capture the recorded calls into a HIP graph on the plan's device and instantiate it (an open
- * fork is joined first).  Allocates the device workspace of the plan's many-vector calls (one slice
+ * fork is joined first).  Consecutive one-vector calls outside a fork that read the same x (and norm), and
+ * whose outputs no other of them reads or writes, are captured as one grouped call where
+ * qvx_qmatmul_group runs one launch (the same bits).  Allocates the device workspace of the plan's many-vector calls (one slice
  * shared by the calls in order, disjoint slices for the calls of one fork), freed with the plan. */
 int qvx_plan_instantiate(qvx_plan* plan);
 /* Replay the graph on `stream` (stream-ordered, asynchronous).  Not instantiated -> QVX_E_STATE. */

@@ -66,7 +66,8 @@ bool launch_dequant16(uint32_t t, const void* src, uint16_t* dst, size_t n, bool
 int launch_quantize_act_q8(const uint16_t* X, int M, int K, int8_t* q, float* scale, int32_t* qsum,
                            hipStream_t s);
 void launch_zero(float* p, size_t n, hipStream_t s);
-bool launch_gemv_group(const GemvMember* m, int n, const float* X, int cols, const GemvEpi& epi, hipStream_t s);
+bool launch_gemv_group(const GemvMember* m, int n, const float* X, int cols, const GemvEpi& epi, hipStream_t s, bool dry);
+bool launch_gemv_vgroup(const GemvMember* m, int n, const float* X, int cols, hipStream_t s, bool dry);
 size_t gemv_many_ws_bytes(int nvec, int rows, int cols, size_t row_bytes);
 int gemv_many_supported(int cols, size_t row_bytes);
 bool launch_gemv_q4k_many(const void* w, const float* X, float* Y, const float* bias, int nvec, int rows, int cols,
@@ -104,6 +105,7 @@ struct qvx_plan {
     int cnt_n = 0;
   };
   std::vector<Call> calls;
+  std::vector<Call> runs;  // what qvx_plan_instantiate makes of them: runs of one-vector calls on one x grouped
   void* ws = nullptr;  // device workspace of the recorded calls, allocated by qvx_plan_instantiate
   int device = 0;
   int open_group = -1;  // the fork being recorded, -1 if none
@@ -552,12 +554,18 @@ static int group_members(float* const* d_out, const void* const* d_w, const uint
   return QVX_OK;
 }
 
-// One launch for the members when the grouped kernel takes them all, else one qmatmul (or
-// qmatmul_n_rmsnorm) each.
-static int gemv_group(const GemvMember* m, int k, const float* x, int cols, const GemvEpi& epi, hipStream_t s) {
+// One launch for the members when a grouped kernel takes them all (dry: only says whether one would).
+static bool gemv_grouped(const GemvMember* m, int k, const float* x, int cols, const GemvEpi& epi, hipStream_t s,
+                         bool dry) {
   bool fast = cols > 0 && aligned16(x);
   for (int i = 0; i < k; ++i) fast = fast && aligned16(m[i].w) && m[i].row_bytes % 16 == 0;
-  if (fast && launch_gemv_group(m, k, x, cols, epi, s)) return hip_status();
+  if (!fast) return false;
+  return launch_gemv_group(m, k, x, cols, epi, s, dry) || (!epi.flags() && launch_gemv_vgroup(m, k, x, cols, s, dry));
+}
+
+// A grouped call: one launch, else one qmatmul (or qmatmul_n_rmsnorm) each.
+static int gemv_group(const GemvMember* m, int k, const float* x, int cols, const GemvEpi& epi, hipStream_t s) {
+  if (gemv_grouped(m, k, x, cols, epi, s, false)) return hip_status();
   for (int i = 0; i < k; ++i)
     if (int rc = gemv(m[i].y, m[i].w, m[i].type, x, 1, m[i].rows, cols, s, epi); rc != QVX_OK) return rc;
   return QVX_OK;
@@ -828,13 +836,14 @@ static int run_call(const qvx_plan& plan, const qvx_plan::Call& c, hipStream_t s
 // bytes the plan needs.
 static size_t plan_ws_layout(qvx_plan& plan) {
   size_t total = 0;
-  for (size_t i = 0; i < plan.calls.size();) {
-    const int g = plan.calls[i].group;
+  auto& calls = plan.runs;
+  for (size_t i = 0; i < calls.size();) {
+    const int g = calls[i].group;
     size_t n = 1;
-    while (g >= 0 && i + n < plan.calls.size() && plan.calls[i + n].group == g) ++n;
+    while (g >= 0 && i + n < calls.size() && calls[i + n].group == g) ++n;
     size_t off = 0;
     for (size_t k = i; k < i + n; ++k) {
-      auto& c = plan.calls[k];
+      auto& c = calls[k];
       c.ws_off = c.ws_bytes = 0;
       c.cnt_off = 0;
       c.cnt_n = 0;
@@ -854,12 +863,61 @@ static size_t plan_ws_layout(qvx_plan& plan) {
     if (off > total) total = off;
     i += n;
   }
-  for (auto& c : plan.calls) {
+  for (auto& c : calls) {
     if (!c.cnt_n) continue;
     c.cnt_off = total;
     total += ((size_t)c.cnt_n * 4 + 255) & ~(size_t)255;
   }
   return total;
+}
+
+// Whether [p, p + n) and [q, q + m) share a byte.
+static bool overlap(const void* p, size_t n, const void* q, size_t m) {
+  const auto a = reinterpret_cast<uintptr_t>(p), b = reinterpret_cast<uintptr_t>(q);
+  return a < b + m && b < a + n;
+}
+
+// The plan's calls with each run of consecutive one-vector products of one x (the decoder's q / k / v and
+// gate / up, recorded one by one) as one grouped call, where a grouped kernel takes the run: each output
+// is its own call's bits (qvx_qmatmul_group).  Calls of a fork stay as they are, and so does a call whose
+// output another member of the run reads or writes.
+static std::vector<qvx_plan::Call> plan_runs(const std::vector<qvx_plan::Call>& calls) {
+  std::vector<qvx_plan::Call> out;
+  const auto single = [](const qvx_plan::Call& c) {
+    return c.members.empty() && c.group < 0 && c.nvec == 1 && c.cols > 0 && !c.epi.swiglu && !c.epi.bias;
+  };
+  for (size_t i = 0; i < calls.size();) {
+    const auto& c = calls[i];
+    std::vector<GemvMember> m;
+    size_t j = i;
+    for (; j < calls.size() && m.size() < QVX_GROUP_MAX && single(calls[j]); ++j) {
+      const auto& d = calls[j];
+      if (d.X != c.X || d.cols != c.cols || d.epi.norm_w != c.epi.norm_w || d.epi.eps != c.epi.eps) break;
+      const TypeInfo* ti = type_info(d.type);
+      const GemvMember e{d.w, d.out, d.type, d.rows, (size_t)(d.cols / (int)ti->block) * ti->bytes};
+      const size_t ob = (size_t)d.rows * 4, wb = (size_t)d.rows * e.row_bytes, xb = (size_t)d.cols * 4;
+      bool clash = overlap(d.out, ob, d.X, xb) || (d.epi.norm_w && overlap(d.out, ob, d.epi.norm_w, xb));
+      for (const auto& o : m)
+        clash = clash || overlap(d.out, ob, o.y, (size_t)o.rows * 4) || overlap(d.out, ob, o.w, o.rows * o.row_bytes) ||
+                overlap(o.y, (size_t)o.rows * 4, d.w, wb);
+      if (clash) break;
+      m.push_back(e);
+      if (m.size() > 1 && !gemv_grouped(m.data(), (int)m.size(), c.X, c.cols, c.epi, nullptr, true)) {
+        m.pop_back();
+        break;
+      }
+    }
+    if (m.size() < 2) {
+      out.push_back(c);
+      ++i;
+      continue;
+    }
+    qvx_plan::Call g{nullptr, nullptr, 0, c.X, 1, 0, c.cols, -1, c.epi, {}};
+    g.members = std::move(m);
+    i += g.members.size();
+    out.push_back(std::move(g));
+  }
+  return out;
 }
 
 int qvx_plan_add_qmatmul_group(qvx_plan* plan, float* const* d_out, const void* const* d_w, const uint32_t* types,
@@ -923,7 +981,7 @@ int qvx_plan_size(const qvx_plan* plan) { return plan ? (int)plan->calls.size() 
 
 int qvx_plan_run_eager(const qvx_plan* plan, void* stream) {
   if (!plan) return QVX_E_NULL;
-  for (const auto& c : plan->calls)
+  for (const auto& c : plan->exec ? plan->runs : plan->calls)
     if (int rc = run_call(*plan, c, as_stream(stream)); rc != QVX_OK) return rc;
   return QVX_OK;
 }
@@ -933,7 +991,7 @@ int qvx_plan_run_eager(const qvx_plan* plan, void* stream) {
 // joined back into `cs` after the group.
 static int plan_record(const qvx_plan* plan, hipStream_t cs, std::vector<hipStream_t>& side,
                        std::vector<hipEvent_t>& events) {
-  const auto& calls = plan->calls;
+  const auto& calls = plan->runs;
   auto event = [&](hipEvent_t* e) {
     if (hipEventCreateWithFlags(e, hipEventDisableTiming) != hipSuccess) return false;
     events.push_back(*e);
@@ -979,6 +1037,11 @@ int qvx_plan_instantiate(qvx_plan* plan) {
   plan->open_group = -1;
   DeviceGuard guard(plan->device);
   if (!guard.ok) return QVX_E_HIP;
+  try {
+    plan->runs = plan_runs(plan->calls);
+  } catch (const std::bad_alloc&) {
+    return QVX_E_HIP;
+  }
   if (const size_t wsb = plan_ws_layout(*plan)) {
     if (hipMalloc(&plan->ws, wsb) != hipSuccess) {
       plan->ws = nullptr;

@@ -1131,8 +1131,9 @@ int gemv_mxj_supported(int cols) {
 // on the matrix-core kernel and at most one Q6_K member on the VALU kernel, all 16-byte aligned
 // with 16-byte row pitches (the operands the standalone fast kernels take), optionally on
 // rmsnorm(x) (epi.norm_w; no SwiGLU).  Returns false, having launched nothing, when a member or the
-// epilogue is outside that set: the caller then runs the members one by one.
-bool launch_gemv_group(const GemvMember* m, int n, const float* X, int cols, const GemvEpi& epi, hipStream_t s) {
+// epilogue is outside that set: the caller then runs the members one by one.  dry: only says whether it
+// would take the group.
+bool launch_gemv_group(const GemvMember* m, int n, const float* X, int cols, const GemvEpi& epi, hipStream_t s, bool dry) {
   if (n < 1 || gemv_mx_max_nv(cols) < 1 || (cols / 256 * 32 + 1023) / 1024 > 2) return false;
   if (epi.swiglu || !mx_epi_supported(epi, 0, cols)) return false;
   GroupArgs a{};
@@ -1161,6 +1162,7 @@ bool launch_gemv_group(const GemvMember* m, int n, const float* X, int cols, con
     }
   }
   if (a.nmx == 0) return false;
+  if (dry) return true;
   const bool tpt1 = (cols / 256 * 32 + 1023) / 1024 <= 1;
   if (epi.norm_w)
     return tpt1 ? launch_group_tpt<1, true>(X, cols, a, nwg, per_group, epi, s)

@@ -155,3 +155,54 @@ def test_int_batch_in_plan_and_capture(cuda):
         cuda.cuda.synchronize()
         np.testing.assert_array_equal(f32bits(out.cpu().numpy()), want)
         np.testing.assert_array_equal(f32bits(cap.cpu().numpy()), want)
+
+
+# Grouped one-vector products of one type: rows per lane group 1, 2, 3-4 and more (chunks), members smaller than
+# a workgroup's groups, short rows (several groups a wave), rows of several waves with two conversion tasks.
+GROUP_CASES = [(qvx.Q8_0, 4096, [4096, 4096, 4096]), (qvx.Q8_0, 512, [40, 7, 300]), (qvx.Q8_0, 4096, [11008, 11008]),
+               (qvx.Q4_0, 11008, [1000, 33, 1, 64]), (qvx.Q4_0, 1024, [20000, 17]), (qvx.Q5_0, 4096, [1024, 1024]),
+               (qvx.Q5_K, 2048, [515, 2048]), (qvx.Q6_K, 4096, [1024, 4096]), (qvx.Q6_K, 14336, [100, 300])]
+
+
+@pytest.mark.parametrize("t,cols,rows", GROUP_CASES)
+def test_same_type_group_matches_members(cuda, t, cols, rows):
+    rng = np.random.default_rng(cols + sum(rows))
+    ws = [dev(cuda, random_weight(t, r, cols, rng)) for r in rows]
+    x = dev(cuda, rng.standard_normal((1, cols)).astype(np.float32))
+    outs = [cuda.full((r,), float("nan"), dtype=cuda.float32, device="cuda") for r in rows]
+    st = cuda.cuda.current_stream().cuda_stream
+    assert qvx.qmatmul_group([o.data_ptr() for o in outs], [w.data_ptr() for w in ws], [t] * len(rows), rows,
+                             x.data_ptr(), cols, st) == qvx.OK
+    for o, w, r in zip(outs, ws, rows):
+        np.testing.assert_array_equal(f32bits(o.cpu().numpy()), f32bits(_run(cuda, w, t, x, r, cols)[0].cpu().numpy()))
+
+
+@pytest.mark.parametrize("t", [qvx.Q8_0, qvx.Q4_K])
+def test_plan_groups_only_independent_calls(cuda, t):
+    """A plan whose consecutive calls share x (grouped when instantiated), then write what the next reads, or
+    write one output twice: the replay gives the calls' results in order, every time."""
+    from qorvix_amd import decode
+    rng = np.random.default_rng(t)
+    n = 512
+    w = [decode.DevWeight(dev(cuda, random_weight(t, n, n, rng, scale=1e-3)), t, n, n) for _ in range(4)]
+    x0 = dev(cuda, rng.standard_normal((1, n)).astype(np.float32))
+    x = x0.clone()
+    a, b, c = (cuda.zeros((1, n), dtype=cuda.float32, device="cuda") for _ in range(3))
+    steps = [(a, 0, x), (b, 1, x), (c, 2, x), (x, 3, x), (a, 1, x), (a, 2, x), (b, 0, a)]
+    plan = decode.Plan()
+    for out, i, src in steps:
+        plan.add(out, w[i], src, 1)
+    assert len(plan) == len(steps)
+    plan.instantiate()
+    st = cuda.cuda.current_stream().cuda_stream
+    want = {k: v.clone() for k, v in zip("xabc", (x0, a, b, c))}
+    name = {id(x): "x", id(a): "a", id(b): "b", id(c): "c"}
+    for out, i, src in steps:
+        want[name[id(out)]] = _run(cuda, w[i].data, t, want[name[id(src)]].clone(), n, n)
+    for run in (plan.launch, plan.launch, plan.run_eager):
+        x.copy_(x0)
+        run(st)
+        cuda.cuda.synchronize()
+        for k, v in zip("xabc", (x, a, b, c)):
+            np.testing.assert_array_equal(f32bits(v.cpu().numpy()), f32bits(want[k].cpu().numpy()))
+    plan.close()
