@@ -103,16 +103,17 @@ int qvx_qmatmul(float* d_out, const void* d_w, uint32_t type, const float* d_x, 
 
 /* out[v * rows + r] for v < n_vec.  Replaces qmatmulN (qmatmul.cpp:64-115).  Each output is
  * bit-identical to qvx_qmatmul on that vector, as the reference promises (qmatmul.hpp:31-32).
- * Q4_K batches of 12 vectors or more on weights of >= 32 Mi elements, and of 24 or more on smaller
- * ones, on the one-vector kernel's shapes (cols a multiple of 256 up to 32768, aligned operands) run
- * on a many-vector form: the activations are converted once into a
- * stream-ordered temporary from the library's pool (nvec * cols * 2.25 bytes, plus 2 KiB per 32-row
- * tile and K range for batches up to 32 vectors), then the weights are streamed once per 64 vectors
- * (once per 16 up to 32 vectors) -- the reference's "dequantize each block once for all nVec dot
- * products" (qmatmul.hpp:24-32); smaller batches stream them once per 8 vectors and allocate
- * nothing, except on rows of >= 8192 elements from 5 to 23 vectors and on weights of <= 4 Mi elements
- * from 12 to 23, which stream them once per 16 on a split form whose K ranges are spread over
- * workgroups (a temporary of rows/32 * KQ * 1 or 2 KiB for the range partials; KQ = 4 or 16 ranges).
+ * Q4_K batches on the one-vector kernel's shapes (cols a multiple of 256 up to 32768, aligned operands)
+ * convert the activations once into a stream-ordered temporary from the library's pool (nvec * cols * 2.25
+ * bytes) and then stream the weights
+ *   - once per 16 vectors: 9 to 32 vectors (23 on rows of < 2048 elements); 8 to 64 on up to 8192 rows of >=
+ *     2048 elements; 5 to 64 on rows of >= 8192 elements (where rows of > 22528 elements take 8 a pass); with
+ *     a norm or SwiGLU folded in (below) 6 to 256 on up to 8192 rows, from 8 or 9 on more;
+ *   - once per 64 vectors: larger batches -- the reference's "dequantize each block once for all nVec dot
+ *     products" (qmatmul.hpp:24-32).
+ * Smaller batches stream them once per 8 vectors (once per call up to 3) and allocate nothing, and so do, on
+ * a capturing stream, those below 24 vectors (12 on weights of >= 32 Mi or <= 4 Mi elements, 5 on rows of >=
+ * 8192 elements).
  * Q6_K batches of 3 vectors and of 5 or more, of 4 on weights of >= 8192 rows or columns and of 2
  * on weights of >= 65536 rows, with cols a multiple of 2048, stream the weights once per 16 vectors
  * (per 4 or 8 when the call has at most that many) on a matrix-core form whose K range is split over
@@ -136,8 +137,8 @@ int qvx_qmatmul_n(float* d_out, const void* d_w, uint32_t type, const float* d_X
  * qvx_qmatmul_n): the reference's wmatmulBias / wmatmulNBias (runtime/include/qorvix/runtime/
  * weights.hpp:58-80), the bias added after the product in fp32, so each output is the bit pattern of
  * qvx_qmatmul_n's output plus bias[r].  The arguments and checks of qvx_qmatmul_n.  The Q4_K batches
- * qvx_qmatmul_n runs on its many-vector form (above) add the bias in its epilogue; other
- * calls run the product, then one bias-add launch. */
+ * that stream the weights once per 64 vectors, the converted Q8_0 / Q4_0 / Q5_0 batches and the fp32-activation
+ * kernels' larger batches add the bias in their store; other calls run the product, then one bias-add launch. */
 int qvx_qmatmul_n_bias(float* d_out, const void* d_w, uint32_t type, const float* d_X, const float* d_bias,
                        int n_vec, int rows, int cols, void* stream);
 

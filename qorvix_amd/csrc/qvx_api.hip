@@ -52,9 +52,6 @@ void launch_read16(const void* src, size_t n16, uint32_t* flag, hipStream_t s);
 bool qgemm_deq_supported(uint32_t t, const void* w, const uint16_t* X, int K, int N, size_t row_bytes);
 int q4k_plan_desc(int M, int N, int K, int cus, int* desc, int cap);
 bool gemv_q6s_route(int nvec, int rows, int cols, size_t row_bytes, size_t* ws_bytes);
-bool gemv_q4s_route(int nvec, int rows, int cols, size_t row_bytes, size_t* ws_bytes);
-bool launch_gemv_q4s(const void* w, const float* X, float* Y, const float* bias, int nvec, int rows, int cols,
-                     size_t row_bytes, void* ws, hipStream_t s);
 bool launch_gemv_q6s(const void* w, const float* X, float* Y, int nvec, int rows, int cols, size_t row_bytes,
                      void* ws, hipStream_t s, uint32_t* cnt);
 int gemv_q6s_counters(int nvec, int rows, int cols);
@@ -68,6 +65,9 @@ int launch_quantize_act_q8(const uint16_t* X, int M, int K, int8_t* q, float* sc
 void launch_zero(float* p, size_t n, hipStream_t s);
 bool launch_gemv_group(const GemvMember* m, int n, const float* X, int cols, const GemvEpi& epi, hipStream_t s, bool dry);
 bool launch_gemv_vgroup(const GemvMember* m, int n, const float* X, int cols, hipStream_t s, bool dry);
+size_t gemv_q4b_ws_bytes(int nvec, int cols);
+bool launch_gemv_q4b(const void* w, const float* X, float* Y, int nvec, int rows, int cols, size_t row_bytes,
+                     const GemvEpi& epi, void* ws, hipStream_t s);
 size_t gemv_many_ws_bytes(int nvec, int rows, int cols, size_t row_bytes);
 int gemv_many_supported(int cols, size_t row_bytes);
 bool launch_gemv_q4k_many(const void* w, const float* X, float* Y, const float* bias, int nvec, int rows, int cols,
@@ -101,6 +101,7 @@ struct qvx_plan {
     GemvEpi epi;  // fused RMSNorm / SwiGLU (rows = the weight's rows: 2 ffn for SwiGLU)
     std::vector<GemvMember> members;  // non-empty: a grouped call over X (nvec 1), out / w / type / rows unused
     size_t ws_off = 0, ws_bytes = 0;  // its slice of the plan's workspace (forms that take one)
+    bool converted = false;           // the call before left its activations converted at ws_off
     size_t cnt_off = 0;               // its zeroed counters (cnt_n), a slice no other call shares
     int cnt_n = 0;
   };
@@ -233,19 +234,34 @@ int gemv_unfused(float* out, const void* w, uint32_t type, const float* X, int n
   return rc;
 }
 
-// out = W . x per vector, optionally with the activations normalised (epi.norm_w) and / or the
-// interleaved gate|up rows gated (epi.swiglu: rows / 2 outputs a vector).  The argument checks are
-// the plain operator's.
-// Whether a Q4_K batch takes the split form (k_gemv_q4s) rather than the many-vector form or chunks
-// of 8 on the one-vector / batched forms.  Measured on MI355X (graph-replayed): it wins on long rows
-// from 5 vectors (4096 x 14336 at 8: 20.5 against 26.0 us, at 16: 28.8 against 34.0 on the
-// many-vector form; at 4: 20.1 against 17.1) and on small weights from 12 (1024 x 4096 at 16: 12.7
-// against 17.6), up to 23 vectors; on 4096-element rows of larger weights the other forms are faster
-// (14336 x 4096 at 8: 17.7 against 14.3).  Its fixed cost (a conversion per workgroup, the partial
-// sums' launch) is ~9 us.
-inline bool q4s_batch(int nvec, int rows, int cols) {
-  if (nvec > 23) return false;
-  return (cols >= 8192 && nvec >= 5) || ((int64_t)rows * cols <= ((int64_t)4 << 20) && nvec >= 12);
+// Whether a Q4_K batch takes the form on converted activations (k_gemv_q4b) rather than the many-vector form
+// or chunks of 8 on the one-vector / batched forms.  Its conversion is a launch of ~3 us (which a plan's
+// call on the activations of the call before it does without).  Measured on MI355X, graph-replayed over
+// distinct weights and activations, conversion included: on rows of >= 8192 elements from 5 vectors (4096 x
+// 14336 at 4: 17.7 against 19.1 us, at 5: 20.5 -> 19.1, at 16: 29.8 -> 24.2, at 64: 117 -> 67); from 8 on up to
+// 8192 rows of >= 2048 (4096 x 4096: 9.7 -> 9.1, 1024 x 4096: 9.4 -> 7.5; at 7 8.8 against 9); from 9 on others
+// (14336 x 4096 at 8 15.1 against 16, at 16: 23.7 -> 19.2; 8192 x 1024 at 9: 9.2 -> 7.8); to 64 where the
+// many-vector form's waves are few (4096 x 4096: 40.7 -> 28.6), to 32 on more rows (14336 x 4096 at 32: 36.4 ->
+// 32.2, at 64 49 against 57) and to 23 on short rows (8192 x 1024 at 24 12.1 against 12.2).  With a norm or
+// SwiGLU folded in the batched form's conversion is longer: from 6 vectors on up to 8192 rows (6144 x 4096:
+// 13.8 -> 11.5), from 8 on more rows of >= 4096 (28672 x 4096 at 6 24.3 against 25.2, at 8: 26.7 -> 25.2), from
+// 9 on others (11264 x 2048 at 8 10.9 against 11.6, at 9: 16.2 -> 13.2), and no many-vector form takes over.
+inline bool q4b_batch(int nvec, int rows, int cols, const GemvEpi& epi) {
+  if (epi.flags()) return nvec >= (rows <= 8192 ? 6 : cols >= 4096 ? 8 : 9) && nvec <= 256;
+  if (cols >= 8192) return nvec >= 5 && nvec <= 64;
+  if (cols < 2048) return nvec >= 9 && nvec <= 23;
+  return rows <= 8192 ? nvec >= 8 && nvec <= 64 : nvec >= 9 && nvec <= 32;
+}
+
+// Whether a call that is being captured, with no workspace of its own, may put a temporary's allocation into
+// the graph.  The integer form never does; of the Q4_K batches those from 12 vectors (24 on weights between 4
+// and 32 Mi elements) and those of 5 or more on long rows do, where the chunked forms would read the weights
+// several times over (4096 x 14336 at 16: 20 against ~50 us), and the smaller ones keep the chunked forms,
+// which take none; a call with a norm or SwiGLU folded in never does.
+inline bool captured_temp(bool q4b, int nvec, int rows, int cols, const GemvEpi& epi) {
+  if (!q4b || epi.flags()) return false;
+  return many_batch(nvec, rows, cols) || cols >= 8192 ||
+         (nvec >= 12 && (int64_t)rows * cols <= ((int64_t)4 << 20));
 }
 
 // Q6_K batches with the RMSNorm prologue: the standalone norm (the engine's canonical sum of squares
@@ -259,7 +275,7 @@ inline bool q6_norm_batched(int nvec, int rows, int cols) {
 }
 
 // The forms that take a workspace, and the bytes of the one a call takes (0: none).
-enum WsForm { WS_NONE, WS_MANY, WS_Q4S, WS_Q6S, WS_Q6S_NORM, WS_INT };
+enum WsForm { WS_NONE, WS_MANY, WS_Q6S, WS_Q6S_NORM, WS_INT, WS_Q4B };
 inline WsForm ws_route(uint32_t type, int nvec, int rows, int cols, size_t row_bytes, bool fast, const GemvEpi& epi,
                        size_t* bytes) {
   *bytes = 0;
@@ -267,6 +283,10 @@ inline WsForm ws_route(uint32_t type, int nvec, int rows, int cols, size_t row_b
   if (!epi.flags()) {
     *bytes = gemv_int_ws_bytes(type, nvec, rows, cols, row_bytes);
     if (*bytes) return WS_INT;
+  }
+  if (type == T_Q4_K && q4b_batch(nvec, rows, cols, epi) && (epi.flags() == 0 || mx_epi_supported(epi, rows, cols))) {
+    *bytes = gemv_q4b_ws_bytes(nvec, cols);
+    if (*bytes) return WS_Q4B;
   }
   if (epi.flags()) {
     if (type == T_Q6_K && epi.flags() == EPI_NORM && q6_norm_batched(nvec, rows, cols) &&
@@ -278,7 +298,6 @@ inline WsForm ws_route(uint32_t type, int nvec, int rows, int cols, size_t row_b
     return WS_NONE;
   }
   if (type == T_Q4_K) {
-    if (q4s_batch(nvec, rows, cols) && gemv_q4s_route(nvec, rows, cols, row_bytes, bytes)) return WS_Q4S;
     if (many_batch(nvec, rows, cols) && gemv_many_supported(cols, row_bytes)) {
       *bytes = gemv_many_ws_bytes(nvec, rows, cols, row_bytes);
       return WS_MANY;
@@ -291,6 +310,10 @@ inline WsForm ws_route(uint32_t type, int nvec, int rows, int cols, size_t row_b
   *bytes = 0;
   return WS_NONE;
 }
+
+// out = W . x per vector, optionally with the activations normalised (epi.norm_w) and / or the
+// interleaved gate|up rows gated (epi.swiglu: rows / 2 outputs a vector).  The argument checks are
+// the plain operator's.
 int gemv(float* out, const void* w, uint32_t type, const float* X, int nvec, int rows, int cols, hipStream_t s,
          const GemvEpi& epi) {
   const TypeInfo* ti = nullptr;
@@ -315,8 +338,9 @@ int gemv(float* out, const void* w, uint32_t type, const float* X, int nvec, int
   //  * Q4_K batches of 12-24 vectors or more (many_batch; encoder and prefill sizes): activations
   //    converted once, the weights streamed once per 64 vectors, bit-identical per vector to the
   //    one-vector kernel (k_gemv_q4k_many), with the bias added in its epilogue.
-  //  * smaller Q4_K batches (q4s_batch): the K ranges split over workgroups (k_gemv_q4s), bit-identical
-  //    per vector to the one-vector kernel, the bias added in its sum launch;
+  //  * smaller Q4_K batches (q4b_batch): activations converted once, the batched form's tiles for 16 vectors
+  //    a launch (k_gemv_q4b), bit-identical per vector to the one-vector kernel; a bias is added after; a
+  //    capturing stream keeps the chunked forms where they are cheap (captured_temp);
   //  * Q6_K batches (q6_batched): the matrix-core form with the K range split over workgroups
   //    (k_gemv_q6s), bit-identical per vector to the VALU kernel; a bias is added after;
   //  * Q8_0 / Q4_0 / Q5_0 batches: activations converted once, then the matrix-core form with the VALU
@@ -327,7 +351,8 @@ int gemv(float* out, const void* w, uint32_t type, const float* X, int nvec, int
   size_t need = 0;
   if (const WsForm form = ws_route(type, nvec, rows, cols, row_bytes, fast, epi, &need); form != WS_NONE) {
     const bool own = epi.ws && epi.ws_bytes >= need;
-    const bool none = epi.no_alloc || (form == WS_INT && !own && stream_capturing(s));
+    const bool none = epi.no_alloc || (!own && (form == WS_INT || form == WS_Q4B) && stream_capturing(s) &&
+                                       !captured_temp(form == WS_Q4B, nvec, rows, cols, epi));
     void* ws = own ? epi.ws : none ? nullptr : gemm_temp_alloc(need, s);
     if (ws) {
       uint32_t* cnt = own && epi.cnt_n >= gemv_q6s_counters(nvec, rows, cols) ? epi.cnt : nullptr;
@@ -340,13 +365,13 @@ int gemv(float* out, const void* w, uint32_t type, const float* X, int nvec, int
                              s, cnt);
       } else {
         ok = form == WS_MANY ? launch_gemv_q4k_many(w, X, out, epi.bias, nvec, rows, cols, row_bytes, ws, s)
+             : form == WS_Q4B ? launch_gemv_q4b(w, X, out, nvec, rows, cols, row_bytes, epi, ws, s)
              : form == WS_INT ? launch_gemv_int(type, w, X, out, epi.bias, nvec, rows, cols, row_bytes, ws, s)
-             : form == WS_Q4S ? launch_gemv_q4s(w, X, out, epi.bias, nvec, rows, cols, row_bytes, ws, s)
                               : launch_gemv_q6s(w, X, out, nvec, rows, cols, row_bytes, ws, s, cnt);
       }
       if (!own) gemm_temp_free(ws, s);
       if (!ok) return refused();
-      if (form == WS_Q6S && epi.bias) launch_add_bias(out, epi.bias, nvec, rows, s);
+      if ((form == WS_Q6S || form == WS_Q4B) && epi.bias) launch_add_bias(out, epi.bias, nvec, rows, s);
       return hip_status();
     }
   }
@@ -821,6 +846,7 @@ static int run_call(const qvx_plan& plan, const qvx_plan::Call& c, hipStream_t s
   if (plan.ws && c.ws_bytes) {
     epi.ws = static_cast<uint8_t*>(plan.ws) + c.ws_off;
     epi.ws_bytes = c.ws_bytes;
+    epi.converted = c.converted;
   }
   if (plan.ws && c.cnt_n) {
     epi.cnt = reinterpret_cast<uint32_t*>(static_cast<uint8_t*>(plan.ws) + c.cnt_off);
@@ -829,13 +855,19 @@ static int run_call(const qvx_plan& plan, const qvx_plan::Call& c, hipStream_t s
   return gemv(c.out, c.w, c.type, c.X, c.nvec, c.rows, c.cols, s, epi);
 }
 
+// Whether [p, p + n) and [q, q + m) share a byte.
+static bool overlap(const void* p, size_t n, const void* q, size_t m) {
+  const auto a = reinterpret_cast<uintptr_t>(p), b = reinterpret_cast<uintptr_t>(q);
+  return a < b + m && b < a + n;
+}
+
 // Lays out the plan's workspace: each call whose form takes a workspace gets a 256-byte aligned
 // slice; calls in order share offset 0, the calls of one fork (which run concurrently) get disjoint
 // slices.  After them, each call that can use tile counters gets its own slice of them (zeroed by
 // qvx_plan_instantiate; the kernels leave them zero, so no other data may share them).  Returns the
 // bytes the plan needs.
 static size_t plan_ws_layout(qvx_plan& plan) {
-  size_t total = 0;
+  size_t total = 0, last_q4b = ~size_t(0) - 1;
   auto& calls = plan.runs;
   for (size_t i = 0; i < calls.size();) {
     const int g = calls[i].group;
@@ -845,6 +877,7 @@ static size_t plan_ws_layout(qvx_plan& plan) {
     for (size_t k = i; k < i + n; ++k) {
       auto& c = calls[k];
       c.ws_off = c.ws_bytes = 0;
+      c.converted = false;
       c.cnt_off = 0;
       c.cnt_n = 0;
       if (!c.members.empty() || c.cols <= 0 || c.rows <= 0) continue;
@@ -857,6 +890,16 @@ static size_t plan_ws_layout(qvx_plan& plan) {
       if (form == WS_NONE) continue;
       c.ws_off = off;
       c.ws_bytes = need;
+      // A batch on the same activations as the call right before it, in order, reads that call's converted
+      // ones (both slices start at 0) unless that call's output lies over them.
+      if (form == WS_Q4B && g < 0 && k > 0 && last_q4b == k - 1) {
+        const auto& d = calls[k - 1];
+        const size_t xb = (size_t)c.nvec * c.cols * 4, ob = (size_t)d.nvec * (d.epi.swiglu ? d.rows / 2 : d.rows) * 4;
+        c.converted = d.X == c.X && d.nvec == c.nvec && d.cols == c.cols && d.epi.norm_w == c.epi.norm_w &&
+                      d.epi.eps == c.epi.eps && !overlap(d.out, ob, c.X, xb) &&
+                      !(c.epi.norm_w && overlap(d.out, ob, c.epi.norm_w, (size_t)c.cols * 4));
+      }
+      if (form == WS_Q4B && g < 0) last_q4b = k;
       off += (need + 255) & ~(size_t)255;
       if (form == WS_Q6S || form == WS_Q6S_NORM) c.cnt_n = gemv_q6s_counters(c.nvec, c.rows, c.cols);
     }
@@ -869,12 +912,6 @@ static size_t plan_ws_layout(qvx_plan& plan) {
     total += ((size_t)c.cnt_n * 4 + 255) & ~(size_t)255;
   }
   return total;
-}
-
-// Whether [p, p + n) and [q, q + m) share a byte.
-static bool overlap(const void* p, size_t n, const void* q, size_t m) {
-  const auto a = reinterpret_cast<uintptr_t>(p), b = reinterpret_cast<uintptr_t>(q);
-  return a < b + m && b < a + n;
 }
 
 // The plan's calls with each run of consecutive one-vector products of one x (the decoder's q / k / v and

@@ -546,13 +546,26 @@ __device__ inline void q4k_group_scales(const u32x4& hd, int c, float& sca, floa
   mnb = (float)(sm >> 24);
 }
 
+// The 6-bit scales and mins of a Q4_K header as bytes: sc[i], mn[i] hold those of sub-blocks 4i .. 4i + 3.
+struct ScBytes {
+  uint32_t sc[2], mn[2];
+};
+__device__ inline ScBytes q4k_scales(const u32x4& hd) {
+  ScBytes r;
+  r.sc[0] = hd.y & 0x3F3F3F3Fu;
+  r.mn[0] = hd.z & 0x3F3F3F3Fu;
+  r.sc[1] = (hd.w & 0x0F0F0F0Fu) | ((hd.y >> 2) & 0x30303030u);
+  r.mn[1] = ((hd.w >> 4) & 0x0F0F0F0Fu) | ((hd.z >> 2) & 0x30303030u);
+  return r;
+}
+
 // One tile's MFMAs and fold: header hd and codes qq (this lane's row j = lane%16, K block
 // r4 = lane/16), A fragments af[sb] of the super-block's eight sub-blocks, activation records
 // mf[2c + e] of group c for vectors 2 r4 + e.  acc[e][c] += the group's term, for both vectors.
 // Group c of the tile: A fragments a0 / a1 of sub-blocks 2c / 2c+1, records m0 / m1 of vectors
 // 2 r4 / 2 r4 + 1 ([sx, Qa, Qb, ...]).
 template <typename MT>
-__device__ inline void mxb_fold_group(int c, const u32x4& hd, const u32x2& q, const u32x2& a0, const u32x2& a1,
+__device__ inline void mxb_fold_group(int c, const u32x4& hd, const ScBytes& sc, const u32x2& q, const u32x2& a0, const u32x2& a1,
                                       const MT& m0, const MT& m1, float (&acc)[2][4]) {
   const float d = f16lo(hd.x), dmin = f16hi(hd.x);
   const u32x2 bl = {q.x & 0x0F0F0F0Fu, q.y & 0x0F0F0F0Fu};
@@ -562,14 +575,17 @@ __device__ inline void mxb_fold_group(int c, const u32x4& hd, const u32x2& q, co
       __builtin_amdgcn_mfma_i32_16x16x32_i8(__builtin_bit_cast(long, a0), __builtin_bit_cast(long, bl), zero, 0, 0, 0);
   const v4i db =
       __builtin_amdgcn_mfma_i32_16x16x32_i8(__builtin_bit_cast(long, a1), __builtin_bit_cast(long, bh), zero, 0, 0, 0);
-  float sca, scb16, mna, mnb;
-  q4k_group_scales(hd, c, sca, scb16, mna, mnb);
+  // v_cvt_f32_ubyte of bytes 2c, 2c+1 of the eight
+  const uint32_t sw = sc.sc[c >> 1] >> (16 * (c & 1)), mw = sc.mn[c >> 1] >> (16 * (c & 1));
+  const float sca = (float)(sw & 0xFFu), scb = (float)((sw >> 8) & 0xFFu);
+  const float mna = (float)(mw & 0xFFu), mnb = (float)((mw >> 8) & 0xFFu);
 #pragma unroll
   for (int e = 0; e < 2; ++e) {
     const MT mt = e == 0 ? m0 : m1;
-    const int ta = (int)((uint32_t)da[2 * e] << 7) + da[2 * e + 1];                      // sum n q, sub-block 2c
-    const int tb = (int)((((uint32_t)db[2 * e] << 7) + (uint32_t)db[2 * e + 1]) << 4);  // 16 sum n q, 2c+1
-    const float t = __builtin_fmaf((float)tb, scb16, (float)ta * sca);
+    const int ta = (int)((uint32_t)da[2 * e] << 7) + da[2 * e + 1];  // sum n q, sub-block 2c
+    // the one-vector kernel takes 16 sum n q and sc / 16 here: the same product, exactly
+    const int tb = (int)((uint32_t)db[2 * e] << 7) + db[2 * e + 1];  // sum n q, sub-block 2c+1
+    const float t = __builtin_fmaf((float)tb, scb, (float)ta * sca);
     const float w = __builtin_fmaf(__uint_as_float(mt.z), mnb, __uint_as_float(mt.y) * mna);
     acc[e][c] = __builtin_fmaf(__builtin_fmaf(d, t, -dmin * w), __uint_as_float(mt.x), acc[e][c]);
   }
@@ -578,8 +594,9 @@ __device__ inline void mxb_fold_group(int c, const u32x4& hd, const u32x2& q, co
 template <typename MT>
 __device__ inline void mxb_fold(const u32x4& hd, const u32x2 (&qq)[4], const u32x2 (&af)[8], const MT (&mf)[8],
                                 float (&acc)[2][4]) {
+  const ScBytes sc = q4k_scales(hd);
 #pragma unroll
-  for (int c = 0; c < 4; ++c) mxb_fold_group(c, hd, qq[c], af[2 * c], af[2 * c + 1], mf[2 * c], mf[2 * c + 1], acc);
+  for (int c = 0; c < 4; ++c) mxb_fold_group(c, hd, sc, qq[c], af[2 * c], af[2 * c + 1], mf[2 * c], mf[2 * c + 1], acc);
 }
 
 // EPI as for k_gemv_mx.
@@ -831,11 +848,12 @@ __global__ __launch_bounds__(1024) void k_gemv_mxj(const uint8_t* __restrict__ W
     if (NEXT_X) mxj_load<NVT>(X, cols, nv, order((U) + 1), lane, x);                                 \
     if (NEXT_COPY) mx_issue(rsrc, off, order((U) + 2), stage + ((U) & 1) * kTileBytes);              \
     mxj_read_half(1, fa, ma, a1, m1);                                                                \
-    mxb_fold_group(0, hd, qq[0], a0[0], a0[1], m0[0], m0[1], acc);                                   \
-    mxb_fold_group(1, hd, qq[1], a0[2], a0[3], m0[2], m0[3], acc);                                   \
+    const ScBytes sc = q4k_scales(hd);                                                               \
+    mxb_fold_group(0, hd, sc, qq[0], a0[0], a0[1], m0[0], m0[1], acc);                               \
+    mxb_fold_group(1, hd, sc, qq[1], a0[2], a0[3], m0[2], m0[3], acc);                               \
     lds_wait8(a1, m1);                                                                               \
-    mxb_fold_group(2, hd, qq[2], a1[0], a1[1], m1[0], m1[1], acc);                                   \
-    mxb_fold_group(3, hd, qq[3], a1[2], a1[3], m1[2], m1[3], acc);                                   \
+    mxb_fold_group(2, hd, sc, qq[2], a1[0], a1[1], m1[0], m1[1], acc);                               \
+    mxb_fold_group(3, hd, sc, qq[3], a1[2], a1[3], m1[2], m1[3], acc);                               \
   }
 
   if (nu >= 2) {
@@ -877,6 +895,192 @@ __global__ __launch_bounds__(1024) void k_gemv_mxj(const uint8_t* __restrict__ W
 
 constexpr int kCUs = 256;
 constexpr size_t kLdsMax = kLdsPerCU;
+
+// ---- batched form on converted activations: up to 16 vectors a launch ----------------------------
+// The batched form's tiles, fold and geometry (so its outputs are the one-vector kernel's bits too), with
+// the activations converted once by a launch of their own instead of by every workgroup: at 8 vectors of
+// 4096 the conversion held a workgroup's first tile copy back by ~5 us.  The fragments stay in global
+// memory (L2): a wave reads the 512 bytes a sub-block and 8 vectors one super-block ahead of their use,
+// each register quad requested again as soon as its MFMAs are issued, so LDS holds only the records
+// (copied once a workgroup, 512 bytes a super-block and 8 vectors) and the tile ring, whatever K, and one
+// pass over the weights serves 16 vectors.  Bound by the fold's VALU work, ~185 instructions a tile, wave and
+// super-block at 8 vectors (the 15-bit products' scales, minimums and float sums, whose order is fixed), not
+// by memory.  Measured on MI355X, graph-replayed over distinct weights, without the conversion's ~3 us: 4096 x
+// 4096 5.7 us at 8 vectors and 6.9 at 16 (9.4 and 18.5 on the forms that convert in every workgroup), 14336 x
+// 4096 12.3 and 16.2 (14.1 and 23.4 on the batched and the many-vector form), 4096 x 14336 13.0 and 17.4 (20.8
+// and 29.2 with the K ranges split over workgroups and summed by a second launch), 1024 x 4096 4.8 and 5.8 (9.1
+// and 12.9).
+//
+// Workspace: a part for every launch's nt <= nt0 tiles of 8 vectors, one after another: fragments
+// [s][t][group c][lane] x 16 bytes (the lane's 8 bytes of sub-blocks 2c and 2c + 1), then records
+// [s][t][c][vector] x 16 bytes (sx, Qa, Qb, unused).
+__host__ __device__ inline size_t q4b_frag_bytes(int nt, int nsb) { return (size_t)nsb * nt * 4096; }
+__host__ __device__ inline size_t q4b_rec_bytes(int nt, int nsb) { return ((size_t)nsb * nt * 512 + 1023) & ~(size_t)1023; }
+
+// One workgroup a vector; vectors past nvec get zero fragments and records.  NORM: rmsnorm(x, NW, eps) is
+// converted (cols % 512 == 0).
+template <bool NORM>
+__global__ __launch_bounds__(512) void k_q4b_conv(const float* __restrict__ X, int nvec, int cols, int nt0,
+                                                  uint8_t* __restrict__ ws, const float* __restrict__ NW, float eps) {
+  __shared__ __attribute__((aligned(16))) float sqp[NORM ? kNormMaxChunks : 4];
+  const int nsb = cols / 256, ntask = nsb * 32, tid = threadIdx.x, v = blockIdx.x;
+  const int part0 = v / (8 * nt0), vl = v - part0 * 8 * nt0, nt = min(nt0, (nvec - part0 * 8 * nt0 + 7) / 8);
+  uint8_t* frag = ws + part0 * (q4b_frag_bytes(nt0, nsb) + q4b_rec_bytes(nt0, nsb));
+  uint8_t* rec = frag + q4b_frag_bytes(nt, nsb);
+  const float4* xv = reinterpret_cast<const float4*>(X + (size_t)min(v, nvec - 1) * cols);
+  float scale = 1.0f;
+  if constexpr (NORM) {
+    for (int t0 = tid & ~63; t0 < ntask; t0 += 512) {  // whole waves: a chunk is 64 tasks
+      const int t = t0 + (tid & 63);
+      const float sq = wave_sum64(norm_sq8(xv[2 * t], xv[2 * t + 1]));
+      if ((tid & 63) == 0) norm_store(lds_addr(sqp) + 4u * (uint32_t)(t0 >> 6), sq);
+    }
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    __builtin_amdgcn_s_barrier();
+    scale = norm_scale(lds_addr(sqp), cols / kNormChunk, cols, eps);
+  }
+  for (int t0 = tid & ~31; t0 < ntask; t0 += 512) {  // 32 tasks a super-block: whole groups of 8 lanes
+    const int t = t0 + (tid & 31);
+    float4 x0 = xv[2 * t], x1 = xv[2 * t + 1];
+    if (v >= nvec) x0 = x1 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if constexpr (NORM)
+      if (v < nvec)
+        norm_apply(x0, x1, scale, reinterpret_cast<const float4*>(NW)[2 * t], reinterpret_cast<const float4*>(NW)[2 * t + 1]);
+    const XQ8 q = mx_quantize(x0, x1);
+    const int s = t >> 5, g = (t >> 3) & 3, part = t & 7, hi = part >> 2, kg = part & 3;
+    const size_t st = (size_t)s * nt + (vl >> 3);
+    uint8_t* f = frag + (st * 4 + g) * 1024 + (16 * kg + 2 * (vl & 7)) * 16 + 8 * hi;
+    *reinterpret_cast<uint2*>(f) = make_uint2(q.h0, q.h1);       // row 2v: qh
+    *reinterpret_cast<uint2*>(f + 16) = make_uint2(q.l0, q.l1);  // row 2v + 1: ql
+    float* m = reinterpret_cast<float*>(rec + ((st * 4 + g) * 8 + (vl & 7)) * 16);
+    if (part == 0) m[0] = q.sx, m[1] = (float)q.sq;
+    if (part == 4) m[2] = (float)q.sq, m[3] = 0.0f;
+  }
+}
+
+template <int NT, int EPI>
+__global__ __launch_bounds__(1024) void k_gemv_q4b(const uint8_t* __restrict__ W, const uint8_t* __restrict__ frag,
+                                                   const uint8_t* __restrict__ rec, float* __restrict__ Y, int rows,
+                                                   int nv, MxGeo geo) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];  // the records
+  __shared__ __attribute__((aligned(16))) uint8_t ring[16 * 2 * kTileBytes];
+  const int nsb = geo.nsb, TQ = geo.TQ, KQ = geo.KQ;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  QVX_LDS uint8_t* stage = (QVX_LDS uint8_t*)(ring + wave * 2 * kTileBytes);
+  const int b = blockIdx.x;
+  const int rb = b * geo.base + geo.unit * min(b, geo.rem), cnt = geo.base + (b < geo.rem ? geo.unit : 0);
+  const int tq = wave % TQ, kq = wave / TQ;
+  const int s0 = kq * nsb / KQ, s1 = (kq + 1) * nsb / KQ, nu = s1 - s0;
+  const SbOrder order(kq, KQ, s0, s1);
+
+  // 1. the records' copies, the first super-block's fragments, the first two tiles
+  {
+    const uint32_t nb = (uint32_t)(nsb * NT * 512);
+    const __amdgpu_buffer_rsrc_t rr = __builtin_amdgcn_make_buffer_rsrc((void*)rec, (short)0, (int)nb, (int)kRsrcWord3);
+    for (uint32_t k = (uint32_t)wave * 1024u; k < nb; k += 16u * 1024u)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rr, (QVX_LDS uint8_t*)lds + k, 16, 16u * (uint32_t)lane, k, 0, 0);
+  }
+  const u32x4* fl = reinterpret_cast<const u32x4*>(frag) + lane;
+  u32x4 a[NT][4];
+  {
+    const int s = nu > 0 ? order(0) : s0;
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int t = 0; t < NT; ++t) a[t][c] = fl[((s * NT + t) * 4 + c) * 64];
+  }
+  const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(W + (size_t)rb * geo.row_bytes), (short)0, (int)((uint32_t)cnt * geo.row_bytes), (int)kRsrcWord3);
+  uint32_t off[3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const uint32_t p = k < 2 ? (uint32_t)(1024 * k + 16 * lane) : (uint32_t)(2048 + 4 * lane);
+    const uint32_t r = p / (uint32_t)kSB, c = p - (uint32_t)kSB * r;
+    off[k] = __umul24(16u * (uint32_t)tq + r, geo.row_bytes) + c;
+  }
+#pragma unroll
+  for (int u = 0; u < 2; ++u) mx_issue(rsrc, off, nu > 0 ? order(min(u, nu - 1)) : s0, stage + u * kTileBytes);
+  wait_vm<6>();  // this wave's records: everything before the tiles
+  __builtin_amdgcn_s_barrier();
+
+  // 2. tiles
+  const int j = lane & 15, r4 = lane >> 4;  // B column (tile row) and K block; D rows 4 r4..4 r4+3
+  const uint32_t b_hd = kSB * j, b_q = kSB * j + 16 + 8 * r4;
+  const uint32_t rec_base = lds_addr(lds) + 32u * (uint32_t)r4;  // vectors 2 r4, 2 r4 + 1 of a tile
+  const uint32_t stage_base = (uint32_t)(uintptr_t)stage;
+  float acc[NT][2][4];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) acc[t][e][c] = 0.0f;
+
+  for (int u = 0; u < nu; ++u) {
+    // newer than tile u's copies: at first tile 1's; then the refill and the fragments of the step before
+    // (and older fragments, already used)
+    if (u == 0) wait_vm<3>();
+    else if (u + 1 < nu) wait_vm<3 + 4 * NT>();
+    else wait_vm<4 * NT>();
+    const int s = order(u), sn = order(min(u + 1, nu - 1));
+    const uint32_t st = stage_base + (uint32_t)((u & 1) * kTileBytes);
+    u32x4 hd = lds_read16(st + b_hd);
+    u32x2 q0 = lds_read8(st + b_q), q1 = lds_read8(st + b_q + 32), q2 = lds_read8(st + b_q + 64),
+          q3 = lds_read8(st + b_q + 96);
+    u32x4 m[NT][2];
+    auto read_rec = [&](int c) __attribute__((always_inline)) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        const uint32_t ma = rec_base + (uint32_t)(((s * NT + t) * 4 + c) * 128);
+        m[t][0] = lds_read16(ma);
+        m[t][1] = lds_read16<16>(ma);
+      }
+    };
+    auto wait_rec = [&]() __attribute__((always_inline)) {
+      if constexpr (NT == 1)
+        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(m[0][0]), "+v"(m[0][1])::"memory");
+      else
+        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(m[0][0]), "+v"(m[0][1]), "+v"(m[NT - 1][0]), "+v"(m[NT - 1][1])::"memory");
+    };
+    read_rec(0);
+    lds_wait5(hd, q0, q1, q2, q3);
+    wait_rec();
+    if (u + 2 < nu) mx_issue(rsrc, off, order(u + 2), stage + (u & 1) * kTileBytes);
+    const u32x2 qq[4] = {q0, q1, q2, q3};
+    const ScBytes sc = q4k_scales(hd);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      u32x4 mc[NT][2];
+#pragma unroll
+      for (int t = 0; t < NT; ++t) mc[t][0] = m[t][0], mc[t][1] = m[t][1];
+      if (c < 3) read_rec(c + 1);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        const u32x2 a0 = {a[t][c].x, a[t][c].y}, a1 = {a[t][c].z, a[t][c].w};
+        mxb_fold_group(c, hd, sc, qq[c], a0, a1, mc[t][0], mc[t][1], acc[t]);
+      }
+#pragma unroll
+      for (int t = 0; t < NT; ++t) a[t][c] = fl[((sn * NT + t) * 4 + c) * 64];
+      if (c < 3) wait_rec();
+    }
+  }
+
+  wait_vm<0>();
+
+  // 3. groups as (g0 + g2) + (g1 + g3), then the KQ waves of the tile in wave order
+  __syncthreads();
+  float* red = reinterpret_cast<float*>(ring);  // [tq][kq][v][16]
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int v = 8 * t + 2 * r4 + e;
+      if (v < nv) red[((tq * KQ + kq) * nv + v) * 16 + j] = (acc[t][e][0] + acc[t][e][2]) + (acc[t][e][1] + acc[t][e][3]);
+    }
+  __syncthreads();
+  mx_store<EPI>(red, Y, nv, rows, rb, cnt, TQ, KQ, tid);
+}
 
 template <int NV, int NB, int TPT, int EPI>
 static bool launch_mx(const void* w, const float* X, float* Y, int rows, int cols, const MxGeo& geo, int nwg,
@@ -1089,6 +1293,67 @@ bool launch_gemv_mxj_q4k(const void* w, const float* X, float* Y, int nvec, int 
     case 3: return launch_mxj<3>(wp, X, Y, nvec, rows, cols, geo, nwg, s);
     default: return launch_mxj<4>(wp, X, Y, nvec, rows, cols, geo, nwg, s);
   }
+}
+
+// Vector tiles a launch of the batched form on converted activations takes: 2, or 1 where the records of two
+// would not fit beside the tile ring (0: not this shape).
+static int q4b_tiles(int cols) {
+  if (!gemv_mxj_supported(cols)) return 0;
+  for (int nt = 2; nt >= 1; --nt)
+    if (q4b_rec_bytes(nt, cols / 256) + (size_t)16 * 2 * kTileBytes <= kLdsMax) return nt;
+  return 0;
+}
+
+// Workspace bytes of a call (0: the form does not take the shape).
+size_t gemv_q4b_ws_bytes(int nvec, int cols) {
+  const int nt0 = q4b_tiles(cols), nsb = cols / 256;
+  if (!nt0) return 0;
+  const int parts = (nvec + 8 * nt0 - 1) / (8 * nt0), nt = (nvec - (parts - 1) * 8 * nt0 + 7) / 8;
+  return (parts - 1) * (q4b_frag_bytes(nt0, nsb) + q4b_rec_bytes(nt0, nsb)) + q4b_frag_bytes(nt, nsb) + q4b_rec_bytes(nt, nsb);
+}
+
+template <int NT, int EPI>
+static bool launch_q4b(const uint8_t* w, const uint8_t* frag, const uint8_t* rec, float* Y, int nv, int rows,
+                       const MxGeo& geo, int nwg, hipStream_t s) {
+  auto kern = &k_gemv_q4b<NT, EPI>;
+  const size_t lds = q4b_rec_bytes(NT, geo.nsb);
+  static LdsLimit lim;
+  if (!lds_ready(reinterpret_cast<const void*>(kern), lim, lds)) return false;
+  kern<<<(unsigned)nwg, 1024u, lds, s>>>(w, frag, rec, Y, rows, nv, geo);
+  return true;
+}
+
+// out = W . X (rmsnorm(X), SwiGLU as epi says) for a batch: one conversion launch, then one launch per 16
+// (or 8) vectors; ws holds gemv_q4b_ws_bytes (epi.converted: this X converted already, as the call
+// before on the workspace left it).  Returns false when a launch cannot be configured.
+bool launch_gemv_q4b(const void* w, const float* X, float* Y, int nvec, int rows, int cols, size_t row_bytes,
+                     const GemvEpi& epi, void* ws, hipStream_t s) {
+  const int nt0 = q4b_tiles(cols), nsb = cols / 256;
+  if (nt0 == 0 || row_bytes >= (1u << 24) || !mx_epi_supported(epi, rows, cols)) return false;
+  MxGeo geo{};
+  const int nwg = mx_geometry(rows, cols, row_bytes, geo, epi.swiglu ? 32 : 1);
+  const auto* wb = static_cast<const uint8_t*>(w);
+  auto* frag = static_cast<uint8_t*>(ws);
+  if (!epi.converted) {
+    const unsigned nwv = 8u * (unsigned)((nvec + 7) / 8);
+    if (epi.norm_w) k_q4b_conv<true><<<nwv, 512, 0, s>>>(X, nvec, cols, nt0, frag, epi.norm_w, epi.eps);
+    else k_q4b_conv<false><<<nwv, 512, 0, s>>>(X, nvec, cols, nt0, frag, nullptr, 0.0f);
+  }
+  for (int v0 = 0; v0 < nvec; v0 += 8 * nt0) {
+    const int nv = std::min(8 * nt0, nvec - v0), nt = (nv + 7) / 8;
+    const uint8_t* rec = frag + q4b_frag_bytes(nt, nsb);
+    float* Yv = Y + (size_t)v0 * (epi.swiglu ? rows / 2 : rows);
+    bool ok;
+    if (epi.swiglu)
+      ok = nt == 1 ? launch_q4b<1, EPI_SWIGLU>(wb, frag, rec, Yv, nv, rows, geo, nwg, s)
+                   : launch_q4b<2, EPI_SWIGLU>(wb, frag, rec, Yv, nv, rows, geo, nwg, s);
+    else
+      ok = nt == 1 ? launch_q4b<1, 0>(wb, frag, rec, Yv, nv, rows, geo, nwg, s)
+                   : launch_q4b<2, 0>(wb, frag, rec, Yv, nv, rows, geo, nwg, s);
+    if (!ok) return false;
+    frag += q4b_frag_bytes(nt0, nsb) + q4b_rec_bytes(nt0, nsb);
+  }
+  return true;
 }
 
 // Largest vector count one launch takes for a row of `cols` columns (LDS budget), 0 if the shape
@@ -1545,405 +1810,6 @@ bool launch_gemv_q4k_many_shape(const void* w, const float* X, float* Y, const f
   }
 #undef QVX_MANY_WK
 #undef QVX_MANY
-  return true;
-}
-
-// ---- batched Q4_K with the K range split over workgroups -------------------------------------------
-// qvx_qmatmul_n over Q4_K, NV (8 or 16) vectors a launch, each weight byte streamed once, every output
-// bit-identical to the one-vector kernel's (k_gemv_mx): the many-vector form's arithmetic per group
-// (the same MFMA sums, the same fold), the same chains and the same order of the K ranges.
-//  * Columns: RPC consecutive whole K ranges of mx_geometry (C super-blocks, at most 8), so every
-//    range's chain stays in one workgroup.  Workgroup b (16 waves) owns column b % ncol and the
-//    32-row tiles b / ncol, b / ncol + P, ...  Its items are the column's (super-block, group) pairs,
-//    item i = 4 sbl + c, taken by wave i % 16 (one or two a wave).  A wave's A fragments (sub-blocks
-//    2c and 2c + 1, 16 vectors x qh / ql) are the same for every tile: converted once (mx_quantize,
-//    through LDS, into registers); the records (Qa, Qb for the fold, sx for the chains) stay in LDS.
-//  * Tiles stream through a two-stage LDS ring (32 rows x the column's bytes, copied by
-//    buffer_load_dword ... lds, rows an odd number of dwords apart).  Per tile and item the wave runs
-//    the group's two v_mfma_i32_32x32x32_i8 and the fold V = fma(d, t, -dmin w) per (row, vector)
-//    into LDS; then four threads an output (one a group) run each range's chain A_c = fma(V, sx, A_c)
-//    over its super-blocks in the one-vector kernel's walk order (SbOrder) and add (A0 + A2) +
-//    (A1 + A3) across the quad: the range's partial, stored to the workspace.
-//  * k_q4s_sum adds each output's KQ range partials in order from 0.0f, then the bias.
-struct Q4sGeo {
-  int nsb;     // super-blocks a row
-  int KQ;      // K ranges of the one-vector geometry
-  int RPC;     // ranges a column
-  int ncol;    // columns (KQ / RPC)
-  int ntile;   // 32-row tiles
-  int P;       // workgroups a column
-  int C;       // super-blocks of the widest column (<= 4 IPW)
-  uint32_t row_bytes;
-};
-
-// The range kq's super-blocks [s0, s1) and walk direction (SbOrder: even ranges backward).
-__device__ __host__ inline void q4s_range(int kq, int nsb, int KQ, int& s0, int& s1, bool& back) {
-  s0 = kq * nsb / KQ;
-  s1 = (kq + 1) * nsb / KQ;
-  back = KQ > 1 && !(kq & 1);
-}
-
-// A 16-byte global load whose wait the kernel places itself (q4s_wait_x), before tile 0's copies:
-// the compiler, which does not see those, would otherwise wait for them too at the value's first use.
-typedef float q4s_f4 __attribute__((ext_vector_type(4)));
-__device__ inline q4s_f4 q4s_ldx(const float* p) {
-  q4s_f4 r;
-  asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(r) : "v"(p));
-  return r;
-}
-// Waits until at most N vector memory operations are outstanding; the loaded values are operands,
-// so no use of them moves above the wait.
-template <int N, int K>
-__device__ inline void q4s_wait_x(q4s_f4* a, q4s_f4* b) {
-  if constexpr (K == 1)
-    asm volatile("s_waitcnt vmcnt(%2)" : "+v"(a[0]), "+v"(b[0]) : "n"(N) : "memory");
-  else if constexpr (K == 2)
-    asm volatile("s_waitcnt vmcnt(%4)" : "+v"(a[0]), "+v"(a[1]), "+v"(b[0]), "+v"(b[1]) : "n"(N) : "memory");
-  else
-    asm volatile("s_waitcnt vmcnt(%8)"
-                 : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(b[0]), "+v"(b[1]), "+v"(b[2]), "+v"(b[3])
-                 : "n"(N)
-                 : "memory");
-}
-// s_waitcnt vmcnt(0) that memory accesses cannot move across.
-__device__ inline void q4s_wait_vm0() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-// Workgroup barrier for LDS only (see q6s_lds_barrier).
-__device__ inline void q4s_lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-// Copy global -> LDS, 4 bytes a lane, as inline asm (see q6s_copy4: the kernel waits for its copies
-// itself; the s_nop is the wait state between the M0 write and the copy).
-__device__ inline void q4s_copy4(__amdgpu_buffer_rsrc_t r, uint32_t dst, uint32_t voff, uint32_t soff) {
-  asm volatile("s_nop 0\n\tbuffer_load_dword %0, %1, %2 offen lds" ::"v"(voff), "s"(r), "s"(soff), "{m0}"(dst)
-               : "memory");
-}
-
-// s_waitcnt vmcnt(N) for the N = 0..3 tiles' copies that may stay in flight.
-template <int CPT>
-__device__ inline void q4s_wait_tiles(int n) {
-  switch (n) {
-    case 0: asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); break;
-    case 1: asm volatile("s_waitcnt vmcnt(%0)" ::"n"(CPT) : "memory"); break;
-    case 2: asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * CPT) : "memory"); break;
-    default: asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * CPT) : "memory"); break;
-  }
-}
-
-// LDS plan of a launch: WPC workgroups a CU.  With one, whole 64-dword copies (every wave makes CPT a
-// tile, so the waits can count them) into up to 4 ring stages; with two (8 vectors, one item a wave),
-// the copies stop at the column's end and the ring has 2 stages.
-template <int NV, int IPW, int WPC>
-struct Q4sLds {
-  static constexpr int CMAX = 4 * IPW;                  // super-blocks a column at most
-  static constexpr int NIT = 4 * CMAX;                  // items at most
-  static constexpr int NO = NV * 32;                    // outputs a tile
-  static constexpr int NCP = (36 * CMAX + 63) / 64;     // 64-dword copies a staged row
-  static constexpr int CPT = 2 * NCP;                   // copies a wave a tile
-  static constexpr int SW = (WPC == 1 ? 64 * NCP : 36 * CMAX) + 1;  // LDS dwords a staged row (odd: rows on distinct banks)
-  static constexpr int STAGE = 32 * SW * 4;             // bytes of a ring stage
-  static constexpr int RB = NV == 8 && IPW == 1 ? 2 : 1;  // step-value buffers
-  static constexpr int RES = NIT * NO * 4;              // bytes of one
-  static constexpr int BUDGET = 160 * 1024 / WPC - NIT * 3 * 16 * 4 - 64;  // the CU's share less recq, sxl
-  static constexpr int NSF = (BUDGET - RB * RES) / STAGE;
-  static constexpr int NS = WPC == 2 ? 2 : NSF > 4 ? 4 : NSF;  // ring stages
-  static constexpr int BYTES = NS * STAGE + RB * RES;
-  static_assert(NS >= 2 && BYTES <= BUDGET, "two ring stages at least, within the budget");
-  static_assert(NV * CMAX * 512 <= STAGE + RB * RES, "conversion scratch fits in the last stage + the buffers");
-};
-
-template <int NV, int IPW, int WPC>
-__global__ __launch_bounds__(1024, 4 * WPC) void k_gemv_q4s(const uint8_t* __restrict__ W, const float* __restrict__ X,
-                                                            int rows, int cols, int nv, Q4sGeo geo,
-                                                            float* __restrict__ part) {
-  static_assert(NV == 8 || NV == 16, "8 or 16 vectors a launch");
-  static_assert(IPW == 1 || IPW == 2, "one or two items a wave");
-  static_assert(WPC == 1 || (WPC == 2 && NV == 8 && IPW == 1), "two workgroups a CU: 8 vectors, one item a wave");
-  using L = Q4sLds<NV, IPW, WPC>;
-  constexpr int NIT = L::NIT, NO = L::NO, NCP = L::NCP, SW = L::SW, STAGE = L::STAGE, RB = L::RB, NS = L::NS;
-  constexpr int KV = NV / 2;  // vectors a lane folds
-  __shared__ __attribute__((aligned(16))) uint8_t lds[L::BYTES];
-  __shared__ __attribute__((aligned(16))) float recq[NIT][2][16];  // [item][Qa, Qb][vector]
-  __shared__ float sxl[NIT][NV];                                    // [item][vector]
-  float* res = reinterpret_cast<float*>(lds + NS * STAGE);          // [buffer][item][vector][row]
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int j = lane & 31, h = lane >> 5;
-  const int col = (int)blockIdx.x % geo.ncol, pi = (int)blockIdx.x / geo.ncol;
-  const int ntl = pi < geo.ntile ? (geo.ntile - pi + geo.P - 1) / geo.P : 0;
-  if (ntl == 0) return;  // the whole workgroup
-  int cs0, cs1;          // the column's super-blocks
-  {
-    bool bk;
-    int t0, t1;
-    q4s_range(col * geo.RPC, geo.nsb, geo.KQ, cs0, t0, bk);
-    q4s_range(col * geo.RPC + geo.RPC - 1, geo.nsb, geo.KQ, t1, cs1, bk);
-  }
-  const int C = cs1 - cs0, nit = 4 * C;
-  const uint32_t lds_base = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(QVX_LDS uint8_t*)lds);
-
-  // Copy of the workgroup's jt-th tile into stage s: wave w copies rows 2w, 2w + 1 (rows past the
-  // weight repeat its last row), each as NCP copies of 64 dwords from the column's first byte on --
-  // whole ones with one workgroup a CU (past the column: the row's next bytes, or zeros past the
-  // weight: the buffer's range; every offset is in the checked vector offset), so that every wave
-  // makes CPT copies a tile and the waits can count them; with two, up to the column's end.
-  auto issue = [&](int jt, int s) __attribute__((always_inline)) {
-    const int r0 = (pi + jt * geo.P) * 32, nr = min(32, rows - r0);
-    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(W + (size_t)r0 * geo.row_bytes), (short)0, (int)((uint32_t)nr * geo.row_bytes), (int)kRsrcWord3);
-#pragma unroll
-    for (int rr = 0; rr < 2; ++rr) {
-      const int r = min(2 * wave + rr, nr - 1);
-      const uint32_t vo = (uint32_t)r * geo.row_bytes + (uint32_t)cs0 * 144u + 4u * lane;
-      const uint32_t dst = lds_base + (uint32_t)(s * STAGE + (2 * wave + rr) * SW * 4);
-#pragma unroll
-      for (int i = 0; i < NCP; ++i)
-        if (WPC == 1 || 64 * i + lane < 36 * C) q4s_copy4(rsrc, dst + 256u * i, vo + 256u * i, 0u);
-    }
-  };
-
-  // The activations of the column, every vector, converted once into the last stage + the buffers
-  // (not in use yet) in the many-vector layout -- A fragments [v][sbl][sub-block][qh / ql][32 bytes]
-  // -- and the records into recq / sxl.  Tiles 0..NS-2 are copied during the conversion.
-  constexpr int NTK = NV * L::CMAX * 32 / 1024;  // conversion tasks a thread at most
-  static_assert(NTK == 1 || NTK == 2 || NTK == 4, "one, two or four conversion tasks a thread");
-  uint8_t* fr = lds + (NS - 1) * STAGE;
-  {
-    q4s_f4 y0[NTK], y1[NTK];
-#pragma unroll
-    for (int k = 0; k < NTK; ++k) {
-      const int t = min(tid + 1024 * k, NV * C * 32 - 1);
-      const int v = t / (C * 32), r = t - v * C * 32;  // r: task of the column, 8 elements
-      const float* src = X + (size_t)min(v, nv - 1) * cols + (size_t)cs0 * 256 + 8 * r;
-      y0[k] = q4s_ldx(src);
-      y1[k] = q4s_ldx(src + 4);
-    }
-    q4s_wait_x<0, NTK>(y0, y1);
-    for (int jt = 0; jt < NS - 1 && jt < ntl; ++jt) issue(jt, jt);
-#pragma unroll
-    for (int k = 0; k < NTK; ++k) {
-      if (1024 * k + 64 * wave >= NV * C * 32) break;  // wave-uniform: no task left for this wave
-      const int T = tid + 1024 * k, t = min(T, NV * C * 32 - 1);
-      const int v = t / (C * 32), r = t - v * C * 32;
-      const bool pad = v >= nv;  // padding vectors: zero fragments and records
-      const float4 x0 = pad ? make_float4(0.0f, 0.0f, 0.0f, 0.0f) : make_float4(y0[k].x, y0[k].y, y0[k].z, y0[k].w);
-      const float4 x1 = pad ? make_float4(0.0f, 0.0f, 0.0f, 0.0f) : make_float4(y1[k].x, y1[k].y, y1[k].z, y1[k].w);
-      const XQ8 q = mx_quantize(x0, x1);  // every lane of the wave takes part
-      if (T < NV * C * 32) {
-        const int sbl = r >> 5, g = (r >> 3) & 3, pt = r & 7;
-        const int sub = 2 * g + (pt >> 2), off = 8 * (pt & 3);
-        uint8_t* base = fr + ((v * C + sbl) * 8 + sub) * 64;
-        *reinterpret_cast<uint2*>(base + off) = make_uint2(q.h0, q.h1);
-        *reinterpret_cast<uint2*>(base + 32 + off) = make_uint2(q.l0, q.l1);
-        const int it = 4 * sbl + g;
-        if (pt == 0) {
-          sxl[it][v] = q.sx;
-          recq[it][0][v] = (float)q.sq;
-        }
-        if (pt == 4) recq[it][1][v] = (float)q.sq;
-      }
-    }
-  }
-  q4s_lds_barrier();
-  // a wave's A fragments: lane (row j = (vector j / 2, part j % 2), K half h) of sub-blocks 2c, 2c + 1
-  v4i af[IPW][2];
-#pragma unroll
-  for (int i = 0; i < IPW; ++i) {
-    const int it = wave + 16 * i, sbl = it >> 2, c = it & 3, va = j >> 1;
-#pragma unroll
-    for (int e = 0; e < 2; ++e) {
-      const bool on = it < nit && va < NV;
-      const uint8_t* p = fr + ((min(va, NV - 1) * C + min(sbl, C - 1)) * 8 + 2 * c + e) * 64 + (j & 1) * 32 + 16 * h;
-      const v4i z = {0, 0, 0, 0};
-      af[i][e] = on ? *reinterpret_cast<const v4i*>(p) : z;
-    }
-  }
-  q4s_lds_barrier();  // every wave's fragments are in registers: the last stage and the buffers are free
-
-  auto fold = [&](int s, float* rb) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < IPW; ++i) {
-      const int it = wave + 16 * i;
-      if (it >= nit) break;  // wave-uniform
-      const int sbl = it >> 2, c = it & 3;
-      const uint8_t* rowp = lds + s * STAGE + j * SW * 4 + sbl * 144;
-      const uint32_t* hp = reinterpret_cast<const uint32_t*>(rowp);
-      const uint32_t* qp = reinterpret_cast<const uint32_t*>(rowp + 16 + 32 * c + 16 * h);
-      const u32x4 hd = {hp[0], hp[1], hp[2], hp[3]};
-      const uint32_t q0 = qp[0], q1 = qp[1], q2 = qp[2], q3 = qp[3];
-      const v4i bl = {(int)(q0 & 0x0F0F0F0Fu), (int)(q1 & 0x0F0F0F0Fu), (int)(q2 & 0x0F0F0F0Fu), (int)(q3 & 0x0F0F0F0Fu)};
-      const v4i bh = {(int)((q0 >> 4) & 0x0F0F0F0Fu), (int)((q1 >> 4) & 0x0F0F0F0Fu), (int)((q2 >> 4) & 0x0F0F0F0Fu),
-                      (int)((q3 >> 4) & 0x0F0F0F0Fu)};
-      const i32x16_t lo = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[i][0], bl, i32x16_t{}, 0, 0, 0);
-      const i32x16_t hi = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[i][1], bh, i32x16_t{}, 0, 0, 0);
-      const float d = f16lo(hd.x), dmin = f16hi(hd.x);
-      float sca, scb16, mna, mnb;
-      q4k_group_scales(hd, c, sca, scb16, mna, mnb);
-      const float scb = scb16 * 16.0f;  // see the many-vector form: the same product, rounded once
-#pragma unroll
-      for (int k = 0; k < KV; ++k) {
-        const int e = 4 * (k >> 1) + 2 * (k & 1), v = 4 * (k >> 1) + 2 * h + (k & 1);
-        const int ta = (int)((uint32_t)lo[e] << 7) + lo[e + 1];
-        const int tb = (int)(((uint32_t)hi[e] << 7) + (uint32_t)hi[e + 1]);
-        const float t = __builtin_fmaf((float)tb, scb, (float)ta * sca);
-        const float w = __builtin_fmaf(recq[it][1][v], mnb, recq[it][0][v] * mna);
-        rb[(it * NV + v) * 32 + j] = __builtin_fmaf(d, t, -dmin * w);
-      }
-    }
-  };
-  auto chains = [&](int jt, const float* rb) __attribute__((always_inline)) {
-    const int tile = pi + jt * geo.P;
-#pragma unroll
-    for (int o4 = tid; o4 < 4 * NO; o4 += 1024) {
-      const int o = o4 >> 2, c = o4 & 3, v = o >> 5;
-      for (int q = 0; q < geo.RPC; ++q) {
-        const int kq = col * geo.RPC + q;
-        int s0, s1;
-        bool back;
-        q4s_range(kq, geo.nsb, geo.KQ, s0, s1, back);
-        float A = 0.0f;
-        for (int u = 0; u < s1 - s0; ++u) {
-          const int it = 4 * ((back ? s1 - 1 - u : s0 + u) - cs0) + c;
-          A = __builtin_fmaf(rb[it * NO + o], sxl[it][v], A);
-        }
-        float u2 = A + dppf<0x4E>(A);  // quad_perm [2,3,0,1]: (A0 + A2) on the quad's lanes 0, 2, (A1 + A3) on 1, 3
-        u2 = u2 + dppf<0xB1>(u2);      // quad_perm [1,0,3,2]: (A0 + A2) + (A1 + A3)
-        if (c == 0) part[((size_t)tile * geo.KQ + kq) * NO + o] = u2;
-      }
-    }
-  };
-
-  // Tile jt: wait for its copies (up to NS - 2 later tiles' may stay in flight), then, after the
-  // barrier, copy tile jt + NS - 1 into the stage of tile jt - 1 (read by every wave by now), fold
-  // tile jt into the step values, and form the range partials (8 vectors, one item a wave: of tile
-  // jt - 1 from the other buffer; else of tile jt after a second barrier).
-  for (int jt = 0; jt < ntl; ++jt) {
-    const int s = jt % NS;
-    if constexpr (NS == 2)
-      q4s_wait_vm0();
-    else
-      q4s_wait_tiles<L::CPT>(min(NS - 2, ntl - 1 - jt));
-    q4s_lds_barrier();
-    if (jt + NS - 1 < ntl) issue(jt + NS - 1, (jt + NS - 1) % NS);
-    if constexpr (RB == 2) {
-      if (jt > 0) chains(jt - 1, res + ((jt - 1) & 1) * (L::RES / 4));
-      fold(s, res + (jt & 1) * (L::RES / 4));
-    } else {
-      fold(s, res);
-      q4s_lds_barrier();
-      chains(jt, res);
-    }
-  }
-  if constexpr (RB == 2) {
-    q4s_lds_barrier();
-    chains(ntl - 1, res + ((ntl - 1) & 1) * (L::RES / 4));
-  }
-}
-
-// out[v, r] = the KQ range partials of (v, r) added in order from 0.0f (+ bias[r]).
-template <bool BIAS>
-__global__ __launch_bounds__(256) void k_q4s_sum(const float* __restrict__ part, float* __restrict__ Y,
-                                                 const float* __restrict__ bias, int rows, int nv, int KQ, int NO,
-                                                 int ntile) {
-  const int idx = (int)blockIdx.x * 256 + (int)threadIdx.x;
-  if (idx >= ntile * NO) return;
-  const int tile = idx / NO, o = idx - tile * NO, v = o >> 5, r = tile * 32 + (o & 31);
-  if (v >= nv || r >= rows) return;
-  const float* p = part + (size_t)tile * KQ * NO + o;
-  float sum = 0.0f;
-  for (int k0 = 0; k0 < KQ; k0 += 8) {  // eight partials in flight at a time, added in order
-    float b8[8];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) b8[k] = p[(size_t)min(k0 + k, KQ - 1) * NO];
-#pragma unroll
-    for (int k = 0; k < 8; ++k)
-      if (k0 + k < KQ) sum += b8[k];
-  }
-  Y[(size_t)v * rows + r] = BIAS ? sum + bias[r] : sum;
-}
-
-int device_cus();
-
-// The launch geometry: the one-vector geometry's ranges grouped into columns of >= 4 super-blocks
-// where they can be (and <= 8); false when a range alone is wider than 8 super-blocks.
-static bool q4s_geometry(int rows, int cols, size_t row_bytes, Q4sGeo& g) {
-  if (gemv_many_supported(cols, row_bytes) == 0 || rows <= 0) return false;
-  MxGeo mg{};
-  (void)mx_geometry(rows, cols, row_bytes, mg);
-  g.nsb = cols / 256;
-  g.KQ = mg.KQ;
-  g.ntile = (rows + 31) / 32;
-  g.row_bytes = (uint32_t)row_bytes;
-  auto width = [&](int rpc) {  // widest column of rpc ranges
-    int w = 0;
-    for (int c0 = 0; c0 < g.KQ; c0 += rpc) {
-      int s0, s1, t0, t1;
-      bool b;
-      q4s_range(c0, g.nsb, g.KQ, s0, t0, b);
-      q4s_range(c0 + rpc - 1, g.nsb, g.KQ, t1, s1, b);
-      w = std::max(w, s1 - s0);
-    }
-    return w;
-  };
-  g.RPC = 0;
-  for (int r = 1; r <= g.KQ; ++r) {
-    if (g.KQ % r) continue;
-    const int w = width(r);
-    if (w > 8) break;
-    g.RPC = r;
-    g.C = w;
-    int lo = g.nsb;  // narrowest column
-    for (int c0 = 0; c0 < g.KQ; c0 += r) {
-      int s0, s1, t0, t1;
-      bool b;
-      q4s_range(c0, g.nsb, g.KQ, s0, t0, b);
-      q4s_range(c0 + r - 1, g.nsb, g.KQ, t1, s1, b);
-      lo = std::min(lo, s1 - s0);
-    }
-    if (lo >= 4) break;
-  }
-  if (g.RPC == 0) return false;
-  g.ncol = g.KQ / g.RPC;
-  g.P = std::max(1, std::min(g.ntile, device_cus() / g.ncol));
-  return true;
-}
-
-// 1 if the split Q4_K form takes the shape, and its workspace bytes for nvec vectors (the range
-// partials) through *ws_bytes.
-bool gemv_q4s_route(int nvec, int rows, int cols, size_t row_bytes, size_t* ws_bytes) {
-  Q4sGeo g;
-  if (nvec <= 0 || !q4s_geometry(rows, cols, row_bytes, g)) return false;
-  if (ws_bytes) *ws_bytes = (size_t)g.ntile * g.KQ * (nvec <= 8 ? 8 : 16) * 32 * 4;
-  return true;
-}
-
-// qmatmul_n over Q4_K on the split form, 16 vectors a launch (8 when the whole call has at most 8),
-// each launch followed by the in-order sum of its range partials (and the bias).
-bool launch_gemv_q4s(const void* w, const float* X, float* Y, const float* bias, int nvec, int rows, int cols,
-                     size_t row_bytes, void* ws, hipStream_t s) {
-  Q4sGeo g;
-  if (nvec <= 0 || !ws || !q4s_geometry(rows, cols, row_bytes, g)) return false;
-  const int nvp = nvec <= 8 ? 8 : 16, NO = nvp * 32;
-  const auto* wb = static_cast<const uint8_t*>(w);
-  auto* part = static_cast<float*>(ws);
-  const unsigned grid = (unsigned)(g.ncol * g.P);
-  const bool ipw2 = g.C > 4;
-  for (int v0 = 0; v0 < nvec; v0 += nvp) {
-    const int nv = std::min(nvp, nvec - v0);
-    const float* Xv = X + (size_t)v0 * cols;
-    float* Yv = Y + (size_t)v0 * rows;
-    if (nvp == 8 && !ipw2) {
-      const int P2 = std::max(1, std::min(g.ntile, 2 * device_cus() / g.ncol));
-      Q4sGeo g2 = g;
-      g2.P = P2;
-      k_gemv_q4s<8, 1, 2><<<(unsigned)(g.ncol * P2), 1024, 0, s>>>(wb, Xv, rows, cols, nv, g2, part);
-    } else if (nvp == 8) {
-      k_gemv_q4s<8, 2, 1><<<grid, 1024, 0, s>>>(wb, Xv, rows, cols, nv, g, part);
-    } else {
-      if (ipw2) k_gemv_q4s<16, 2, 1><<<grid, 1024, 0, s>>>(wb, Xv, rows, cols, nv, g, part);
-      else k_gemv_q4s<16, 1, 1><<<grid, 1024, 0, s>>>(wb, Xv, rows, cols, nv, g, part);
-    }
-    const unsigned sg = (unsigned)((g.ntile * NO + 255) / 256);
-    if (bias) k_q4s_sum<true><<<sg, 256, 0, s>>>(part, Yv, bias, rows, nv, g.KQ, NO, g.ntile);
-    else k_q4s_sum<false><<<sg, 256, 0, s>>>(part, Yv, nullptr, rows, nv, g.KQ, NO, g.ntile);
-  }
   return true;
 }
 

@@ -108,6 +108,7 @@ struct GemvEpi {
   size_t ws_bytes = 0;
   uint32_t* cnt = nullptr;  // non-null: cnt_n counters, zero on entry, to be left zero (a plan's)
   int cnt_n = 0;
+  bool converted = false;  // the workspace holds this call's activations as the call before it converted them
   int flags() const { return (norm_w ? EPI_NORM : 0) | (swiglu ? EPI_SWIGLU : 0); }
 };
 

@@ -131,12 +131,13 @@ def test_unaligned_row_pitch_rmsnorm(cuda):
     np.testing.assert_array_equal(f32bits(got.cpu().numpy()), f32bits(want.cpu().numpy()))
 
 
-def test_int_batch_in_plan_and_capture(cuda):
-    """A plan's batch (its workspace made at instantiation) and a captured call (no temporary) give the eager
-    call's bits on every replay."""
+@pytest.mark.parametrize("t,n", [(qvx.Q4_0, 21), (qvx.Q4_K, 9), (qvx.Q4_K, 21)])
+def test_batch_in_plan_and_capture(cuda, t, n):
+    """A plan's batch (its workspace made at instantiation) and a captured call (no temporary, but for the last
+    case) give the eager call's bits on every replay."""
     from qorvix_amd import decode
     rng = np.random.default_rng(11)
-    t, rows, cols, n = qvx.Q4_0, 96, 1024, 21
+    rows, cols = 96, 1024
     w = decode.DevWeight(dev(cuda, random_weight(t, rows, cols, rng)), t, rows, cols)
     X = dev(cuda, rng.standard_normal((n, cols)).astype(np.float32))
     want = f32bits(qvx.qmatmul_t(w.data, t, X, rows, cols).cpu().numpy())
@@ -205,4 +206,59 @@ def test_plan_groups_only_independent_calls(cuda, t):
         cuda.cuda.synchronize()
         for k, v in zip("xabc", (x, a, b, c)):
             np.testing.assert_array_equal(f32bits(v.cpu().numpy()), f32bits(want[k].cpu().numpy()))
+    plan.close()
+
+
+# Q4_K batches on converted activations (k_gemv_q4b): fewer super-blocks than K ranges, ragged rows, several
+# launches with a short last one, one vector tile a launch (rows past 22528), many tiles a workgroup.
+Q4B_CASES = [(1, 256, 9), (33, 512, 17), (4096, 2048, 8), (1000, 2304, 64), (300, 10240, 5), (40, 24576, 20),
+             (70000, 256, 12), (515, 14336, 33), (9000, 4096, 32)]
+
+
+@pytest.mark.parametrize("rows,cols,n", Q4B_CASES)
+def test_q4k_batches_match_single_vectors(cuda, rows, cols, n):
+    _check(cuda, qvx.Q4_K, rows, cols, n, seed=rows + cols + n, bias=True, zero_vec=True)
+
+
+@pytest.mark.parametrize("rows,cols,n", [(64, 512, 6), (320, 4096, 16), (96, 1024, 40), (9216, 1024, 9)])
+def test_q4k_batches_norm_and_swiglu_match_single_vectors(cuda, rows, cols, n):
+    rng = np.random.default_rng(rows + n)
+    w = dev(cuda, random_weight(qvx.Q4_K, rows, cols, rng))
+    X = dev(cuda, rng.standard_normal((n, cols)).astype(np.float32))
+    nw = dev(cuda, (1 + 0.1 * rng.standard_normal(cols)).astype(np.float32))
+    for call in (lambda x: qvx.qmatmul_rmsnorm_t(w, qvx.Q4_K, x, nw, 1e-5, rows, cols),
+                 lambda x: qvx.qmatmul_swiglu_t(w, qvx.Q4_K, x, rows // 2, cols),
+                 lambda x: qvx.qmatmul_swiglu_t(w, qvx.Q4_K, x, rows // 2, cols, norm_w=nw, eps=1e-5)):
+        one = cuda.cat([call(X[i:i + 1].contiguous()) for i in (0, n - 1)])
+        np.testing.assert_array_equal(f32bits(call(X)[[0, n - 1]].cpu().numpy()), f32bits(one.cpu().numpy()))
+
+
+def test_plan_batches_share_only_unchanged_activations(cuda):
+    """Consecutive batches on the same activations share their conversion inside a plan, unless the call
+    between them writes the activations, uses others, or is of another form."""
+    from qorvix_amd import decode
+    rng = np.random.default_rng(21)
+    n, d = 9, 512
+    w = [decode.DevWeight(dev(cuda, random_weight(qvx.Q4_K, d, d, rng, scale=1e-3)), qvx.Q4_K, d, d) for _ in range(3)]
+    v = decode.DevWeight(dev(cuda, random_weight(qvx.Q6_K, 64, d, rng, scale=1e-3)), qvx.Q6_K, 64, d)
+    x0 = dev(cuda, rng.standard_normal((n, d)).astype(np.float32))
+    x, u = x0.clone(), dev(cuda, rng.standard_normal((n, d)).astype(np.float32))
+    outs = [cuda.zeros((n, d), dtype=cuda.float32, device="cuda") for _ in range(5)]
+    ov = cuda.zeros((n, 64), dtype=cuda.float32, device="cuda")
+    steps = [(outs[0], w[0], x), (outs[1], w[1], x), (x, w[2], x), (outs[2], w[0], x), (ov, v, x), (outs[3], w[1], x),
+             (outs[4], w[0], u)]
+    plan = decode.Plan()
+    for o, ww, src in steps:
+        plan.add(o, ww, src, n)
+    plan.instantiate()
+    st = cuda.cuda.current_stream().cuda_stream
+    xa = qvx.qmatmul_t(w[2].data, qvx.Q4_K, x0, d, d)
+    want = [qvx.qmatmul_t(ww.data, ww.type, src, ww.rows, d)
+            for ww, src in ((w[0], x0), (w[1], x0), (w[0], xa), (w[1], xa), (w[0], u), (v, xa))]
+    for run in (plan.launch, plan.launch, plan.run_eager):
+        x.copy_(x0)
+        run(st)
+        cuda.cuda.synchronize()
+        for o, e in zip(outs + [ov, x], want + [xa]):
+            np.testing.assert_array_equal(f32bits(o.cpu().numpy()), f32bits(e.cpu().numpy()))
     plan.close()
