@@ -216,8 +216,9 @@ int qvx_interleave_rows16(void* d_dst, const void* d_a, const void* d_b, uint32_
  * Other types, and Q6_K calls those kernels decline, are dequantised into a stream-ordered 16-bit
  * temporary (fp16, bf16 for QVX_GEMM_BF16; per panel of rows) and multiplied by the plain 16-bit MFMA
  * GEMM of qvx_gemm16.  QVX_GEMM_I8 takes Q4_K only (other types: QVX_E_TYPE).  Grids smaller than
- * the chip (small M) split K across workgroups; the last split of each output tile adds the partial
- * tiles in split order, so every call returns the same bits for the same inputs. */
+ * the chip (small M) split K across workgroups; the partial tiles are added in split order, by a launch of
+ * their own or by the last split of each output tile, so every call returns the same bits for the same
+ * inputs. */
 int qvx_qgemm_f16(float* d_out, const void* d_w, uint32_t type, const uint16_t* d_X, int M,
                   int rows, int cols, int variant, void* stream);
 

@@ -217,6 +217,47 @@ struct TileMap {
   int cols_a, mt_a, base_a, mt_b, base_b;
 };
 
+// Partial tile of a K split for k_split_sum: MT 32-token subtiles (those at or past token M are left out),
+// 16 bytes a thread and four of its rows: part[subtile][e / 4][thread][e % 4].
+template <int MT>
+__device__ __forceinline__ void split_store(const f32x16_t* acc, float* __restrict__ part, int m0, int M, int tid) {
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    if (m0 + 32 * i >= M) break;
+#pragma unroll
+    for (int e4 = 0; e4 < 4; ++e4)
+      reinterpret_cast<float4*>(part)[(4 * i + e4) * 512 + tid] =
+          make_float4(acc[i][4 * e4], acc[i][4 * e4 + 1], acc[i][4 * e4 + 2], acc[i][4 * e4 + 3]);
+  }
+}
+
+// The sums of a K-split launch's partial tiles in split order 0, 1, ..., S-1, stored to Y: a workgroup takes
+// 512 threads' four rows of one tile (grid 4 MT x tiles of BM = 32 MT tokens, numbered as the launch before:
+// column-major, M-tile fastest).
+__global__ __launch_bounds__(512) void k_split_sum(const float* __restrict__ part, float* __restrict__ Y, int M, int N,
+                                                   int S, int mt, int bm) {
+  const int c = blockIdx.x, tile = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
+  const int m = (tile % mt) * bm + 8 * c + 4 * (lane >> 5), n = (tile / mt) * kBN + 32 * (tid >> 6) + (lane & 31);
+  if ((tile % mt) * bm + 32 * (c >> 2) >= M) return;
+  const float4* p = reinterpret_cast<const float4*>(part) + ((size_t)tile * S * (bm / 8) + c) * 512 + tid;
+  const size_t zs = (size_t)(bm / 8) * 512;
+  float4 v = p[0];
+  for (int z0 = 1; z0 < S; z0 += 4) {
+    float4 t[4];
+#pragma unroll
+    for (int z = 0; z < 4; ++z) t[z] = p[(size_t)min(z0 + z, S - 1) * zs];
+#pragma unroll
+    for (int z = 0; z < 4; ++z)
+      if (z0 + z < S) v = make_float4(v.x + t[z].x, v.y + t[z].y, v.z + t[z].z, v.w + t[z].w);
+  }
+  if (n >= N) return;
+  float* y = Y + (size_t)m * N + n;
+  if (m < M) y[0] = v.x;
+  if (m + 1 < M) y[N] = v.y;
+  if (m + 2 < M) y[2 * (size_t)N] = v.z;
+  if (m + 3 < M) y[3 * (size_t)N] = v.w;
+}
+
 }  // namespace gemm
 
 using namespace gemm;
@@ -481,8 +522,13 @@ __global__ __launch_bounds__(512) void k_qgemm_q4k(const uint8_t* __restrict__ W
   if (kb < kb1) slice(kb, b0, b1, a);
   wait_vm<0>();
 
-  // K split: the split that finishes a tile last sums the partials in split order and stores it.
+  // K split: the partials are summed in split order, by the launch after (no counters) or by the split that
+  // finishes a tile last.
   if (gridDim.z > 1) {
+    if (!geo.cnt) {
+      split_store<MT>(acc, geo.part + ((size_t)tile_id * gridDim.z + blockIdx.z) * (MT * 16 * 512), m0, M, tid);
+      return;
+    }
     float v[MT * 16];
 #pragma unroll
     for (int a = 0; a < MT * 16; ++a) v[a] = acc[a >> 4][a & 15];
@@ -1122,6 +1168,10 @@ __global__ __launch_bounds__(512) void k_qgemm_q6k8(const uint8_t* __restrict__ 
   wait_vm<0>();
 
   if (gridDim.z > 1) {
+    if (!geo.cnt) {
+      split_store<MT>(acc, geo.part + ((size_t)tile_id * gridDim.z + blockIdx.z) * (MT * 16 * 512), m0, M, tid);
+      return;
+    }
     float v[MT * 16];
 #pragma unroll
     for (int i = 0; i < MT * 16; ++i) v[i] = acc[i >> 4][i & 15];
@@ -1666,15 +1716,27 @@ struct Q4kPlan {
   Q4kLaunch l[2];
 };
 
+// Whether a K split's partial tiles are summed by a launch of their own (k_split_sum) rather than by the split
+// that finishes a tile last, whose workgroup reads S x 128 KB back alone, ~2.5 us a split.  Measured on MI355X,
+// bf16, conversion of X included: 4096 x 4096 at M = 17 28.3 -> 18.4 us and at 201 31.9 -> 25.5 (8 splits), 1024
+// x 4096 at 201 28.6 -> 20.4, 4096 x 14336 at 201 53.2 -> 46.4; Q6_K 4096 x 14336 at 201 65.3 -> 59.  Of two
+// splits only while the tiles are few: 2048 x 1024 at M = 17 (8 tiles) 17.1 -> 13.3 us, at 400 (32) 19.8 -> 19.0,
+// but 14336 x 4096 at 201 (112) 46.1 against 46.7 and at 400 69.8 against 76.2.
+inline bool split_sum(const Q4kLaunch& L) { return L.splits > 2 || (L.splits == 2 && L.ntiles <= 64); }
+void launch_split_sum(float* out, const float* part, int M, int N, const Q4kLaunch& L, hipStream_t s) {
+  k_split_sum<<<dim3((unsigned)L.bm / 8, (unsigned)L.ntiles), 512, 0, s>>>(part, out, M, N, L.splits, L.tm.mt_a, L.bm);
+}
+
 template <int VAR, int BM>
 bool launch_q4k(float* out, const void* w, const uint16_t* X, int M, int N, int K, const Q4kLaunch& L,
                 float* part, uint32_t* cnt, hipStream_t s) {
   static LdsLimit lim;
   if (!lds_ready(reinterpret_cast<const void*>(&k_qgemm_q4k<VAR, BM>), lim, 0)) return false;
-  if (L.splits > 1 && (!part || !cnt)) return false;
+  if (L.splits > 1 && (!part || (!cnt && !split_sum(L)))) return false;
   const int per = split_per(K / 64, L.splits);
   GemmGeo geo{M, N, K, (uint32_t)(K / 256) * 144u, per, 0x0F0F0F0Fu, 0xF0F0F0F0u, 0x000F000Fu, 0x00F000F0u, part, cnt};
   k_qgemm_q4k<VAR, BM><<<dim3(L.ntiles, 1, L.splits), 512, 0, s>>>(static_cast<const uint8_t*>(w), X, out, geo, L.tm);
+  if (split_sum(L)) launch_split_sum(out, part, M, N, L, s);
   return true;
 }
 
@@ -1709,10 +1771,39 @@ namespace {
 
 inline int cdiv(int a, int b) { return (a + b - 1) / b; }
 
+// K splits of a launch of `tiles` 128-token tiles: powers of two while the grid is below ~200 workgroups and a
+// split keeps `fewest` slices, then the count of no more splits that is estimated to be fastest, or of more (down
+// to one super-block a split) where that is estimated to save another 1.5 us.  The estimate: a round of
+// workgroups costs 4 us and 1 us a slice, the sum 2 us, 0.6 us a split and the partials' write and read at 6
+// TB/s.  Measured on MI355X, bf16, conversion of X included: 4096 x 4096 at M = 257 with 8 splits (384 workgroups)
+// 34.2 us, with 4 28.6; 4096 x 14336 at 257 with 8 72.5, with 5 60.5; 2048 x 1024 at 17 with 2 13.3, with 4 10.9; Q6_K
+// 1024 x 4096 at 201 with 4 29.2, with 8 23.7, with 16 24.7; Q6_K 4096 x 14336 at 17 with 14 49.9, with 28 37.1; but
+// 4096 x 4096 at 17 with 8 18.5, with 16 20.4.  More splits than `fewest` allows only where the partials (at
+// most 256 tiles, 32 MiB) fit the no-allocation scratch beside any copy of X.
+int split_count(int M, int N, int nsl, int tiles, int fewest, int cus) {
+  auto most = [&](int least) {
+    int n = 1;
+    while (tiles * n < 200 * cus / 256 && nsl / (n * 2) >= least) n *= 2;
+    return n;
+  };
+  const int base = most(fewest);
+  const bool deep = tiles <= 64 && (size_t)M * (size_t)nsl <= ((size_t)8 << 20) / 64;
+  double best = 0.0;
+  int pick = 0;
+  for (int pass = 0; pass < 2; ++pass)
+    for (int n = pass ? base + 1 : 1; n <= (pass ? deep ? most(4) : 0 : base); ++n) {
+      const int S = cdiv(nsl, split_per(nsl, n));
+      if (pass && tiles * S > 256) break;
+      const double bytes = (double)S * cdiv(M, 32) * 32 * cdiv(N, kBN) * kBN * 8.0;
+      const double c = cdiv(tiles * S, cus) * (4.0 + split_per(nsl, n)) + (S > 1 ? 2.0 + 0.6 * S + bytes / 6e6 : 0.0);
+      if (!pick || c < best - (pass && S > base ? 1.5 : 0.0)) best = c, pick = S;
+    }
+  return pick;
+}
+
 // Tile plan for an M x N x K launch on `cus` compute units (one 512-thread workgroup fits a CU).
-//  * Grids smaller than the chip: 128-token tiles, splitting K (each split stores its partial tile;
-//    the last split of a tile sums them in split order) only while the grid is below ~200
-//    workgroups.
+//  * Grids smaller than the chip: 128-token tiles, splitting K (split_count; each split stores its partial
+//    tile, summed in split order) only while the grid is below ~200 workgroups.
 //  * Otherwise the cheapest of: a uniform grid of 256-, 192- or 128-token tiles, or two launches,
 //    the first of 256-token tiles from token 0 and the second of 192- or 128-token tiles for the
 //    rest, with two kinds of columns (x columns with a1 + b1 tiles, the others with a2 + b2).  The
@@ -1728,11 +1819,8 @@ void q4k_plan(int M, int N, int K, int cus, Q4kPlan& p) {
   };
   p.n = 1;
   if (nt * cdiv(M, 256) < 224 * cus / 256) {
-    int splits = 1;
     const int tiles = nt * cdiv(M, 128);
-    while (tiles * splits < 200 * cus / 256 && nsl / (splits * 2) >= 8) splits *= 2;
-    const int per = split_per(nsl, splits);
-    p.l[0] = uniform(128, (nsl + per - 1) / per);
+    p.l[0] = uniform(128, split_count(M, N, nsl, tiles, 8, cus));
     return;
   }
   auto cost = [&](int bm, int tiles) { return tiles ? cdiv(tiles, cus) * (bm / 256.0 + 0.05) : 0.0; };
@@ -1788,16 +1876,12 @@ size_t q4k_split_bytes(const Q4kPlan& p) {
   return parts + (((size_t)L.ntiles * 4 + 255) & ~(size_t)255);
 }
 
-// The Q6_K kernel (k_qgemm_q6k8): 128-token tiles, K split while the grid is below ~200 workgroups
-// and each split keeps >= 16 slices (its prologue stages two super-blocks; measured against >= 8
-// and >= 32 on the Llama-3-8B shapes: 4-7 % faster than >= 8 below M = 384, up to 23 % at 384).
+// The Q6_K kernel (k_qgemm_q6k8): 128-token tiles, K split in the same way; a prologue stages two super-blocks,
+// so a split keeps 16 slices unless the estimate says otherwise.
 void q6k8_plan(int M, int N, int K, int cus, Q4kPlan& p) {
-  const int nt = cdiv(N, kBN), nsl = K / 64, tiles = nt * cdiv(M, 128);
-  int splits = 1;
-  while (tiles * splits < 200 * cus / 256 && nsl / (splits * 2) >= 16) splits *= 2;
-  const int per = split_per(nsl, splits);
+  const int nt = cdiv(N, kBN), tiles = nt * cdiv(M, 128);
   p.n = 1;
-  p.l[0] = Q4kLaunch{128, (nsl + per - 1) / per, tiles, TileMap{nt, cdiv(M, 128), 0, 1, 0}};
+  p.l[0] = Q4kLaunch{128, split_count(M, N, K / 64, tiles, 16, cus), tiles, TileMap{nt, cdiv(M, 128), 0, 1, 0}};
 }
 
 // 1 if k_qgemm_q6k8 takes this call: an even number of blocks a row (every row's blocks share one
@@ -1820,13 +1904,14 @@ bool launch_q6k8(float* out, const void* w, const uint16_t* X, int M, int N, int
   const Q4kLaunch& L = p.l[0];
   const size_t sb = q4k_split_bytes(p);
   float* part = sb ? static_cast<float*>(ws) : nullptr;
-  uint32_t* cnt = !sb ? nullptr
+  uint32_t* cnt = !sb || split_sum(L) ? nullptr
                  : scnt ? scnt
                         : reinterpret_cast<uint32_t*>(static_cast<uint8_t*>(ws) + (size_t)L.ntiles * L.splits * 128 * kBN * 4);
   if (L.splits > 1 && !ws) return false;
   Q6kGeo geo{M, N, K, (uint32_t)(K / 256) * 210u, split_per(K / 64, L.splits), 0x0F0F0F0Fu, 0x30303030u,
              0x00FF00FFu, part, cnt};
   k_qgemm_q6k8<VAR><<<dim3(L.ntiles, 1, L.splits), 512, 0, s>>>(static_cast<const uint8_t*>(w), X, out, geo, L.tm);
+  if (split_sum(L)) launch_split_sum(out, part, M, N, L, s);
   return true;
 }
 
@@ -1836,7 +1921,7 @@ bool launch_var(float* out, const void* w, const uint16_t* X, int M, int N, int 
                 uint32_t* scnt, hipStream_t s) {
   const size_t sb = q4k_split_bytes(p);
   float* part = sb ? static_cast<float*>(ws) : nullptr;
-  uint32_t* cnt = !sb ? nullptr
+  uint32_t* cnt = !sb || split_sum(p.l[0]) ? nullptr
                  : scnt ? scnt
                         : reinterpret_cast<uint32_t*>(static_cast<uint8_t*>(ws) +
                                                       (size_t)p.l[0].ntiles * p.l[0].splits * p.l[0].bm * kBN * 4);
@@ -1909,8 +1994,8 @@ int launch_qgemm(float* out, const void* w, uint32_t t, const uint16_t* X, int M
       }
       // the K split's counters: the stream's zeroed block for calls that may allocate, else the
       // temporary's, cleared by the bf16 prepass or a zero kernel
-      uint32_t* scnt = sbytes && !ws ? gemm_stream_counters((size_t)plan.l[0].ntiles, s) : nullptr;
-      const size_t cbytes = sbytes && !scnt ? (((size_t)plan.l[0].ntiles * 4 + 255) & ~(size_t)255) : 0;
+      uint32_t* scnt = sbytes && !ws && !split_sum(plan.l[0]) ? gemm_stream_counters((size_t)plan.l[0].ntiles, s) : nullptr;
+      const size_t cbytes = sbytes && !scnt && !split_sum(plan.l[0]) ? (((size_t)plan.l[0].ntiles * 4 + 255) & ~(size_t)255) : 0;
       float* cnt = cbytes ? reinterpret_cast<float*>(tmp + xbytes + sbytes - cbytes) : nullptr;
       const uint16_t* Xg = X;
       if (variant == VAR_BF16) {
@@ -1981,8 +2066,8 @@ int launch_qgemm(float* out, const void* w, uint32_t t, const uint16_t* X, int M
     uint8_t* split_ws = static_cast<uint8_t*>(tmp) + xbytes;
     // the K split's counters: the stream's zeroed block for calls that may allocate, else the
     // temporary's, cleared by the bf16 prepass or a zero kernel
-    uint32_t* scnt = sbytes && !ws ? gemm_stream_counters((size_t)plan.l[0].ntiles, s) : nullptr;
-    const size_t cbytes = sbytes && !scnt ? (((size_t)plan.l[0].ntiles * 4 + 255) & ~(size_t)255) : 0;
+    uint32_t* scnt = sbytes && !ws && !split_sum(plan.l[0]) ? gemm_stream_counters((size_t)plan.l[0].ntiles, s) : nullptr;
+    const size_t cbytes = sbytes && !scnt && !split_sum(plan.l[0]) ? (((size_t)plan.l[0].ntiles * 4 + 255) & ~(size_t)255) : 0;
     float* cnt = cbytes ? reinterpret_cast<float*>(split_ws + sbytes - cbytes) : nullptr;
     const size_t ncnt4 = cbytes / 16;
     const uint16_t* Xg = X;

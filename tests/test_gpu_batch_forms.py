@@ -262,3 +262,26 @@ def test_plan_batches_share_only_unchanged_activations(cuda):
         for o, e in zip(outs + [ov, x], want + [xa]):
             np.testing.assert_array_equal(f32bits(o.cpu().numpy()), f32bits(e.cpu().numpy()))
     plan.close()
+
+
+# K splits of the prefill GEMM whose partial tiles a launch of their own sums (k_split_sum): 2, 4, 5, 7, 8 and 28
+# splits, a last split shorter than the others, subtiles and rows past M, columns past N.
+@pytest.mark.parametrize("t,M,rows,cols", [(qvx.Q4_K, 17, 2048, 1024), (qvx.Q4_K, 257, 4096, 14336),
+                                           (qvx.Q4_K, 65, 3300, 3328), (qvx.Q4_K, 201, 1001, 4096),
+                                           (qvx.Q4_K, 1, 256, 2304), (qvx.Q6_K, 17, 4096, 14336),
+                                           (qvx.Q6_K, 130, 1001, 4096), (qvx.Q6_K, 97, 300, 512)])
+@pytest.mark.parametrize("variant", [qvx.GEMM_BF16, qvx.GEMM_F16])
+def test_gemm_k_split_sum(cuda, t, M, rows, cols, variant):
+    rng = np.random.default_rng(M + rows)
+    w = dev(cuda, random_weight(t, rows, cols, rng, scale=1e-3))
+    X = dev(cuda, (0.5 * rng.standard_normal((M, cols))).astype(np.float16))
+    out = cuda.full((M + 1, rows), 7.0, dtype=cuda.float32, device="cuda")
+    qvx.qgemm_t(w, t, X, rows, cols, variant, out=out[:M])
+    got = out.cpu().numpy()
+    assert (got[M] == 7.0).all()
+    Wd = oracle.dequantize(t, w.cpu().numpy(), rows * cols).reshape(rows, cols).astype(np.float64)
+    ref = X.cpu().numpy().astype(np.float64) @ Wd.T
+    # each product's operands rounded to 8 or 11 bits, and fp32 sums of `cols` products
+    eps = 2.0 ** (-8 if variant == qvx.GEMM_BF16 else -11)
+    bound = (2 * eps + cols * 2.0 ** -24) * (np.abs(X.cpu().numpy().astype(np.float64)) @ np.abs(Wd).T)
+    assert (np.abs(got[:M] - ref) <= bound).all()
