@@ -113,10 +113,12 @@ __device__ inline void lds_wait_w2(u32x4* r, u32x4* w) {
                  : QVX_R2(r, 0), QVX_R2(r, 2), QVX_R2(r, 4), QVX_R2(r, 6), QVX_R2(w, 0)::"memory");
 }
 
-__device__ inline void lds_wait8_1(u32x4* r, u32x4* w) {
-  asm volatile("s_waitcnt lgkmcnt(0)"
-               : "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(r[3]), "+v"(r[4]), "+v"(r[5]), "+v"(r[6]), "+v"(r[7]),
-                 "+v"(w[0])::"memory");
+// Waits as above for r[0..3], w and a.
+__device__ inline void lds_wait4(u32x4* r, uint32_t& w) {
+  asm volatile("s_waitcnt lgkmcnt(0)" : QVX_R2(r, 0), QVX_R2(r, 2), "+v"(w)::"memory");
+}
+__device__ inline void lds_wait4(u32x4* r, u32x4& a, uint32_t& w) {
+  asm volatile("s_waitcnt lgkmcnt(0)" : QVX_R2(r, 0), QVX_R2(r, 2), "+v"(a), "+v"(w)::"memory");
 }
 
 __device__ inline uint32_t xswz(uint32_t r) { return (r ^ ((r >> 3) & 3u)) & 7u; }
@@ -1199,8 +1201,12 @@ __global__ __launch_bounds__(512) void k_qgemm_q6k8(const uint8_t* __restrict__ 
 // prepass; the weight nibbles are int8 operands as they are.  Per 32-element block b (one Q4_K
 // sub-block) one v_mfma_i32_32x32x32_i8 gives the exact integer dot I = sum q * n, folded as
 //   out += sx * (ds * I - dm * qsum) = I * (sx * ds) - (sx * qsum) * dm
-// (ds = d*sc, dm = dmin*m of the sub-block).  The fold is 4 VALU per output per block, against one
-// MFMA per 1024 outputs: this variant is bound by the fold, not by the matrix cores.
+// (ds = d*sc, dm = dmin*m of the sub-block).  The minimums' part is a matrix product over the blocks,
+// sum_b (sx qsum)[m][b] dm[n][b]: one v_mfma_f32_32x32x2_f32 a 32 x 32 tile adds both blocks of a slice to the
+// accumulators in fp32 FMAs, which leaves 3 VALU per output and block to the fold (conversion, sx * ds, FMA), against
+// one int8 MFMA per 1024 outputs: this variant is bound by the fold, not by the matrix cores.  Measured on MI355X with the
+// minimums on the matrix core, before (4 VALU an output and block) -> after, the conversion of X included: 14336 x 4096 at
+// M = 512 155 -> 130 us, at 2048 543 -> 435; 3000 x 11008 at 1024 214 -> 174; 4096 x 4096 at 128 55 -> 48.5.
 //
 // Workgroup = 256 threads, tile 128 tokens x 256 weight rows; wave w owns rows 64w..64w+63 and all
 // 128 tokens (fp32 accumulators in VGPRs, as the fold updates them).  Per 64-column slice: int8 X
@@ -1272,7 +1278,7 @@ typedef int i32x16_t __attribute__((ext_vector_type(16)));
 __device__ inline uint32_t qswz1(uint32_t r) { return ((r >> 2) ^ (r >> 3)) & 1u; }
 }  // namespace gemm
 
-__global__ __launch_bounds__(256) void k_qgemm_q4k_i8(const uint8_t* __restrict__ W, const int8_t* __restrict__ Q,
+__global__ __launch_bounds__(256, 2) void k_qgemm_q4k_i8(const uint8_t* __restrict__ W, const int8_t* __restrict__ Q,
                                                       const float* __restrict__ SC, float* __restrict__ Y,
                                                       GemmGeo geo) {
   constexpr int BM = kI8BM, MT = BM / 32;
@@ -1351,8 +1357,9 @@ __global__ __launch_bounds__(256) void k_qgemm_q4k_i8(const uint8_t* __restrict_
     q_rel[j] = 4096u + 32u * r + 16u * ((uint32_t)g ^ qswz1(r));
   }
   const uint32_t s_rel = 4u * (uint32_t)(4 * g);  // token 8q + 4g + t of a 32-token tile
+  const uint32_t sq_rel = 4u * (uint32_t)((2 + g) * BM + ln);  // sx * qsum of block g, token ln: the minimums' A operand
 
-  float acc[MT][2][16];
+  f32x16_t acc[MT][2];
 #pragma unroll
   for (int i = 0; i < MT; ++i)
 #pragma unroll
@@ -1370,9 +1377,10 @@ __global__ __launch_bounds__(256) void k_qgemm_q4k_i8(const uint8_t* __restrict_
                    wb = ws_base + (uint32_t)st * WST;
     u32x4 wv[4] = {lds_read16(wb + h_rel[0]), lds_read16(wb + q_rel[0]), lds_read16(wb + h_rel[1]),
                    lds_read16(wb + q_rel[1])};
-    lds_wait<4>(wv);
+    uint32_t sq = lds_read4<0>(sb + sq_rel);
+    lds_wait4(wv, sq);
     const ScaleSel sel = scale_sel(c);
-    float ds[2][2], dm[2][2];  // [h][j]
+    float ds[2][2], dmn[2];  // [h][j]; -dm of block g: the minimums' B operands
     i32x4_t bq[2][2];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
@@ -1382,35 +1390,39 @@ __global__ __launch_bounds__(256) void k_qgemm_q4k_i8(const uint8_t* __restrict_
       const float d = f16lo(hd.x), dmin = f16hi(hd.x);
       ds[0][j] = d * ub(scp, 0);
       ds[1][j] = d * ub(scp, 1);
-      dm[0][j] = dmin * ub(mp, 0);
-      dm[1][j] = dmin * ub(mp, 1);
+      dmn[j] = -dmin * (g ? ub(mp, 1) : ub(mp, 0));
       bq[0][j] = i32x4_t{(int)(qq.x & geo.mask_lo), (int)(qq.y & geo.mask_lo), (int)(qq.z & geo.mask_lo),
                          (int)(qq.w & geo.mask_lo)};
       bq[1][j] = i32x4_t{(int)((qq.x >> 4) & geo.mask_lo), (int)((qq.y >> 4) & geo.mask_lo),
                          (int)((qq.z >> 4) & geo.mask_lo), (int)((qq.w >> 4) & geo.mask_lo)};
     }
+    // The next 32 tokens' minimums are issued behind each tile's first products, so that the matrix core works on
+    // them while the VALU folds.
+    auto minimums = [&](int i) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
+      for (int j = 0; j < 2; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(sq), dmn[j], acc[i][j], 0, 0, 0);
+    };
+    minimums(0);
 #pragma unroll
-      for (int i = 0; i < MT; ++i) {
-        u32x4 av[1] = {lds_read16(xb + a_rel[h] + 2048u * i)};
-        u32x4 sv[8];
+    for (int i = 0; i < MT; ++i) {
 #pragma unroll
-        for (int q4 = 0; q4 < 4; ++q4) {
-          sv[q4] = lds_read16(sb + 4u * (uint32_t)(h * BM + 32 * i + 8 * q4) + s_rel);
-          sv[4 + q4] = lds_read16(sb + 4u * (uint32_t)((2 + h) * BM + 32 * i + 8 * q4) + s_rel);
-        }
-        lds_wait8_1(sv, av);
+      for (int h = 0; h < 2; ++h) {
+        u32x4 av = lds_read16(xb + a_rel[h] + 2048u * i);
+        const uint32_t sa = sb + s_rel + 4u * (uint32_t)(h * BM + 32 * i);
+        u32x4 sv[4] = {lds_read16<0>(sa), lds_read16<32>(sa), lds_read16<64>(sa), lds_read16<96>(sa)};
+        if (h == 0 && i + 1 < MT) sq = lds_read4<0>(sb + sq_rel + 128u * (i + 1));
+        lds_wait4(sv, av, sq);
+        i32x16_t I[2];
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const i32x16_t I = __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(i32x4_t, av[0]), bq[h][j],
-                                                                   i32x16_t{}, 0, 0, 0);
+        for (int j = 0; j < 2; ++j)
+          I[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(i32x4_t, av), bq[h][j], i32x16_t{}, 0, 0, 0);
+        if (h == 0 && i + 1 < MT) minimums(i + 1);
 #pragma unroll
-          for (int e = 0; e < 16; ++e) {
-            const float sx = __uint_as_float(sv[e >> 2][e & 3]), sq = __uint_as_float(sv[4 + (e >> 2)][e & 3]);
-            acc[i][j][e] = __builtin_fmaf((float)I[e], sx * ds[h][j], __builtin_fmaf(-sq, dm[h][j], acc[i][j][e]));
-          }
-        }
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int e = 0; e < 16; ++e)
+            acc[i][j][e] = __builtin_fmaf((float)I[j][e], __uint_as_float(sv[e >> 2][e & 3]) * ds[h][j], acc[i][j][e]);
       }
     }
     wait_vm<0>();

@@ -285,3 +285,26 @@ def test_gemm_k_split_sum(cuda, t, M, rows, cols, variant):
     eps = 2.0 ** (-8 if variant == qvx.GEMM_BF16 else -11)
     bound = (2 * eps + cols * 2.0 ** -24) * (np.abs(X.cpu().numpy().astype(np.float64)) @ np.abs(Wd).T)
     assert (np.abs(got[:M] - ref) <= bound).all()
+
+
+# The int8 prefill GEMM's two parts (integer products on the int8 matrix cores, minimums on the fp32 one), against
+# the quantised operands in fp64: one token, remainders of the 32-token subtiles, 128-token and 256-row tiles, K splits
+# with and without a short last one.
+@pytest.mark.parametrize("M,rows,cols", [(1, 1, 256), (33, 257, 768), (97, 300, 1280), (129, 255, 4096), (512, 513, 1024)])
+def test_gemm_i8_minimums(cuda, M, rows, cols):
+    rng = np.random.default_rng(M + rows)
+    w = random_weight(qvx.Q4_K, rows, cols, rng, scale=1e-3)
+    X = (0.5 * rng.standard_normal((M, cols)) + 0.25).astype(np.float16)  # a mean: the minimums weigh in
+    out = cuda.full((M + 1, rows), 7.0, dtype=cuda.float32, device="cuda")
+    qvx.qgemm_t(dev(cuda, w), qvx.Q4_K, dev(cuda, X), rows, cols, qvx.GEMM_I8, out=out[:M])
+    got = out.cpu().numpy()
+    assert (got[M] == 7.0).all()
+    q, s, _ = oracle.quantize_q8_act(X.astype(np.float32))
+    Xq = q.astype(np.float64) * np.repeat(s.astype(np.float64), 32, axis=1)
+    zero = w.reshape(-1, 144).copy()
+    zero[:, 16:] = 0  # codes 0: the values are -dmin * m
+    Wd = oracle.dequantize(qvx.Q4_K, w, rows * cols).reshape(rows, cols).astype(np.float64)
+    Wm = oracle.dequantize(qvx.Q4_K, zero.reshape(-1), rows * cols).reshape(rows, cols).astype(np.float64)
+    # two fp32 terms a 32-element block, each rounded at most 4 times before it is added
+    bound = (cols / 16 + 8) * 2.0 ** -24 * (np.abs(Xq) @ (np.abs(Wd - Wm) + np.abs(Wm)).T)
+    assert (np.abs(got[:M] - Xq @ Wd.T) <= bound + 1e-30).all()
