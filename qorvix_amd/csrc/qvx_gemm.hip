@@ -1211,7 +1211,8 @@ __global__ __launch_bounds__(512) void k_qgemm_q6k8(const uint8_t* __restrict__ 
 // Workgroup = 256 threads, tile 128 tokens x 256 weight rows; wave w owns rows 64w..64w+63 and all
 // 128 tokens (fp32 accumulators in VGPRs, as the fold updates them).  Per 64-column slice: int8 X
 // (128 x 64 bytes), the tile's scales (4 x 128 floats: sx of both blocks, sx*qsum of both) and the
-// weight headers + group-c quant bytes are copied into LDS (two stages, one slice ahead).
+// weight headers + group-c quant bytes are copied into LDS (two stages, one slice ahead).  A K split's partial
+// tiles are summed as the 16-bit kernels' are (split_sum).
 constexpr int kI8BM = 128;
 
 // Quantiser prepass: one thread per 32-value block of the (tile-padded) M x K activations.  Writes
@@ -1359,13 +1360,13 @@ __global__ __launch_bounds__(256, 2) void k_qgemm_q4k_i8(const uint8_t* __restri
   const uint32_t s_rel = 4u * (uint32_t)(4 * g);  // token 8q + 4g + t of a 32-token tile
   const uint32_t sq_rel = 4u * (uint32_t)((2 + g) * BM + ln);  // sx * qsum of block g, token ln: the minimums' A operand
 
-  f32x16_t acc[MT][2];
+  f32x16_t acc[2][MT];
 #pragma unroll
   for (int i = 0; i < MT; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+      for (int e = 0; e < 16; ++e) acc[j][i][e] = 0.0f;
 
   issue(kb0);
   wait_vm<0>();
@@ -1401,7 +1402,7 @@ __global__ __launch_bounds__(256, 2) void k_qgemm_q4k_i8(const uint8_t* __restri
     auto minimums = [&](int i) {
 #pragma unroll
       for (int j = 0; j < 2; ++j)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(sq), dmn[j], acc[i][j], 0, 0, 0);
+        acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(sq), dmn[j], acc[j][i], 0, 0, 0);
     };
     minimums(0);
 #pragma unroll
@@ -1422,7 +1423,7 @@ __global__ __launch_bounds__(256, 2) void k_qgemm_q4k_i8(const uint8_t* __restri
         for (int j = 0; j < 2; ++j)
 #pragma unroll
           for (int e = 0; e < 16; ++e)
-            acc[i][j][e] = __builtin_fmaf((float)I[j][e], __uint_as_float(sv[e >> 2][e & 3]) * ds[h][j], acc[i][j][e]);
+            acc[j][i][e] = __builtin_fmaf((float)I[j][e], __uint_as_float(sv[e >> 2][e & 3]) * ds[h][j], acc[j][i][e]);
       }
     }
     wait_vm<0>();
@@ -1430,16 +1431,22 @@ __global__ __launch_bounds__(256, 2) void k_qgemm_q4k_i8(const uint8_t* __restri
     __builtin_amdgcn_s_barrier();
   }
 
+  if (gridDim.z > 1 && !geo.cnt) {  // summed by k_split_sum, whose threads hold 32 rows a wave
+    float* part = geo.part + (((size_t)blockIdx.x * ntile + tile) * gridDim.z + blockIdx.z) * (BM * kBN);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) split_store<MT>(acc[j], part, m0, M, (2 * wave + j) * 64 + lane);
+    return;
+  }
   if (gridDim.z > 1) {
     const int t = (int)(blockIdx.y * gridDim.x + blockIdx.x);
     float v[MT * 32];
 #pragma unroll
-    for (int a = 0; a < MT * 32; ++a) v[a] = acc[a >> 5][(a >> 4) & 1][a & 15];
+    for (int a = 0; a < MT * 32; ++a) v[a] = acc[(a >> 4) & 1][a >> 5][a & 15];
     if (!split_k_last<MT * 32, 256>(v, geo.part + (size_t)t * gridDim.z * (MT * 32 * 256), geo.cnt + t,
                                     (int)gridDim.z, (int)blockIdx.z, tid, reinterpret_cast<int*>(xs)))
       return;
 #pragma unroll
-    for (int a = 0; a < MT * 32; ++a) acc[a >> 5][(a >> 4) & 1][a & 15] = v[a];
+    for (int a = 0; a < MT * 32; ++a) acc[(a >> 4) & 1][a >> 5][a & 15] = v[a];
   }
 
 #pragma unroll
@@ -1451,7 +1458,7 @@ __global__ __launch_bounds__(256, 2) void k_qgemm_q4k_i8(const uint8_t* __restri
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
         const int m = m0 + 32 * i + 8 * (e >> 2) + 4 * g + (e & 3);
-        if (m < M) Y[(size_t)m * N + n] = acc[i][j][e];
+        if (m < M) Y[(size_t)m * N + n] = acc[j][i][e];
       }
     }
 }
@@ -1734,7 +1741,10 @@ struct Q4kPlan {
 // x 4096 at 201 28.6 -> 20.4, 4096 x 14336 at 201 53.2 -> 46.4; Q6_K 4096 x 14336 at 201 65.3 -> 59.  Of two
 // splits only while the tiles are few: 2048 x 1024 at M = 17 (8 tiles) 17.1 -> 13.3 us, at 400 (32) 19.8 -> 19.0,
 // but 14336 x 4096 at 201 (112) 46.1 against 46.7 and at 400 69.8 against 76.2.
-inline bool split_sum(const Q4kLaunch& L) { return L.splits > 2 || (L.splits == 2 && L.ntiles <= 64); }
+// The int8 kernel: 4096 x 4096 at M = 17 47 -> 32.5 us and at 128 48.5 -> 38.2 (8 and 8 splits), 4096 x 14336 at 201 99.5 ->
+// 80.8, 1024 x 4096 at 2048 67 -> 58.6; 14336 x 4096 at 512 (two splits of 224 tiles) keeps the one launch, 130.
+inline bool split_sum(int splits, int ntiles) { return splits > 2 || (splits == 2 && ntiles <= 64); }
+inline bool split_sum(const Q4kLaunch& L) { return split_sum(L.splits, L.ntiles); }
 void launch_split_sum(float* out, const float* part, int M, int N, const Q4kLaunch& L, hipStream_t s) {
   k_split_sum<<<dim3((unsigned)L.bm / 8, (unsigned)L.ntiles), 512, 0, s>>>(part, out, M, N, L.splits, L.tm.mt_a, L.bm);
 }
@@ -2111,13 +2121,14 @@ int launch_qgemm(float* out, const void* w, uint32_t t, const uint16_t* X, int M
     const size_t sbytes = (size_t)nsl * ntile * 4 * kI8BM * 4;
     if (sbytes >= (1u << 31)) return -7;
     const size_t pbytes = splits > 1 ? (size_t)tiles * splits * kI8BM * kBN * 4 : 0;
-    const size_t cbytes = splits > 1 ? (((size_t)tiles * 4 + 255) & ~(size_t)255) : 0;
+    const bool sum = split_sum(splits, tiles);
+    const size_t cbytes = splits > 1 && !sum ? (((size_t)tiles * 4 + 255) & ~(size_t)255) : 0;
     uint8_t* qb = static_cast<uint8_t*>(gemm_ws(qbytes + sbytes + pbytes + cbytes, ws, ws_cap, s));
     if (!qb) return no_mem;
     int8_t* q = reinterpret_cast<int8_t*>(qb);
     float* sc = reinterpret_cast<float*>(qb + qbytes);
     float* part = splits > 1 ? reinterpret_cast<float*>(qb + qbytes + sbytes) : nullptr;
-    uint32_t* cnt = splits > 1 ? reinterpret_cast<uint32_t*>(qb + qbytes + sbytes + pbytes) : nullptr;
+    uint32_t* cnt = cbytes ? reinterpret_cast<uint32_t*>(qb + qbytes + sbytes + pbytes) : nullptr;
     const size_t nblk = (size_t)Mpad * (cols / 32);
     k_quant_q8_gemm<<<(unsigned)((nblk + 255) / 256), 256, 0, s>>>(
         X, M, cols, Mpad, q, sc, reinterpret_cast<float4*>(cnt), cbytes / 16);
@@ -2125,6 +2136,8 @@ int launch_qgemm(float* out, const void* w, uint32_t t, const uint16_t* X, int M
                 0x00F000F0u, part, cnt};
     dim3 grid((rows + kBN - 1) / kBN, ntile, splits);
     k_qgemm_q4k_i8<<<grid, 256, 0, s>>>(static_cast<const uint8_t*>(w), q, sc, out, geo);
+    if (sum)
+      k_split_sum<<<dim3(kI8BM / 8, (unsigned)tiles), 512, 0, s>>>(part, out, M, rows, splits, ntile, kI8BM);
     gemm_ws_release(qb, ws, s);
     return 0;
   }
