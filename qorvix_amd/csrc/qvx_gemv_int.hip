@@ -12,8 +12,10 @@
 //    takes Q4_0 as 16 (n - 8) and multiplies by 1/16 at the end: exact scalings by a power of two);
 //  * the same reduction: a balanced pairwise tree over each 64 consecutive slots (over the next power of
 //    two, at least 8, for shorter rows), the 64-slot sums added in order.  The one-vector kernel's
-//    padding lanes add their mirrored last slot times 0, a zero of that slot's sign; here they add -0,
-//    the same sum: a zero sum is -0 only where every slot's is, the last one's included.
+//    padding lanes add their mirrored last slot times 0: a zero of that slot's sign, or NaN where the
+//    slot's sum is not finite (a non-finite scale).  Here padding slots add -0, the same sum (a zero sum is
+//    -0 only where every slot's is, the last one's included), and a padded row's last slot adds its own
+//    sum times 0 to itself.
 #include "qvx_gemv_valu.hpp"
 
 namespace qvx {
@@ -167,6 +169,7 @@ __global__ __launch_bounds__(64 * KS * VT, 2) void k_gemv_int(const uint8_t* __r
   // span / KS slots a wave, nck chunks a part.
   const int span = min(Sp, 64), part = span / KS, nck = part / kC, lck = 31 - __clz(nck), nblk = (S + span - 1) / span;
   const bool many = Sp > 64;
+  const int last = S - (S % span != 0 ? 1 : 0);  // a padded row's last slot, or none: the slots from it on need care
 
   // Copies chunk c (block c / nck) of every part into ring half h, all threads, without a branch: rows
   // and chunks are whole 16-byte pieces, pieces past the row repeat its last one (their slots add
@@ -234,7 +237,7 @@ __global__ __launch_bounds__(64 * KS * VT, 2) void k_gemv_int(const uint8_t* __r
 #pragma unroll
     for (int u = 0; u < kC; ++u) {
       const int s = s0 + u;
-      float p[8];
+      float p[8], f[8];
       const i32x16_t zero = {};
       const i32x16_t C0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(
           A0[u], i32x4_t{(int)c0[0], (int)c0[1], (int)c0[2], (int)c0[3]}, zero, 0, 0, 0);
@@ -249,11 +252,16 @@ __global__ __launch_bounds__(64 * KS * VT, 2) void k_gemv_int(const uint8_t* __r
       for (int k = 0; k < 8; ++k) {  // vector 4 (k/2) + 2g + k%2: accumulators 2k (qh), 2k + 1 (ql)
         const int t0 = (int)(((uint32_t)C0[2 * k] << 7) + (uint32_t)C0[2 * k + 1]);
         const int t1 = (int)(((uint32_t)C1[2 * k] << 7) + (uint32_t)C1[2 * k + 1]);
-        const float f = __builtin_fmaf(e1, (float)t1, e0 * (float)t0);
-        p[k] = f * sx[k];
+        f[k] = __builtin_fmaf(e1, (float)t1, e0 * (float)t0);
+        p[k] = f[k] * sx[k];
         asm volatile("" : "+v"(p[k]));  // rounded before the tree adds it
-        if (s >= S) p[k] = -0.0f;
       }
+      if (s >= last)  // uniform
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          p[k] = s == last && last < S ? __builtin_fmaf(f[k], 0.0f, p[k]) : -0.0f;
+          asm volatile("" : "+v"(p[k]));  // in the branch, not selected on every slot
+        }
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
         if (u == 0) v[k] = p[k];

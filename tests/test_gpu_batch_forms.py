@@ -86,6 +86,30 @@ def test_int_batch_keeps_non_finite_vectors_apart(cuda):
     np.testing.assert_array_equal(f32bits(got[keep]), f32bits(clean[keep]))
 
 
+# Slots a row: 4 of 8, 12 of 16, one whole block of 64, two blocks and 44 of 64.
+@pytest.mark.parametrize("t", [qvx.Q8_0, qvx.Q4_0, qvx.Q5_0])
+@pytest.mark.parametrize("cols", [256, 768, 4096, 11008])
+def test_int_batch_non_finite_scales(cuda, t, cols):
+    """Infinite and NaN block scales, also in a row's last slot (whose sum the padding lanes mirror), give a
+    batch what they give single vectors, and leave other rows as they are."""
+    rng = np.random.default_rng(cols)
+    rows, n = 37, 19
+    nb = qvx.row_bytes(t, cols) // (cols // 32)  # a block starts with its fp16 scale
+    w_np = random_weight(t, rows, cols, rng).reshape(rows, cols // 32, nb)
+    X = dev(cuda, rng.standard_normal((n, cols)).astype(np.float32))
+    clean = _run(cuda, dev(cuda, w_np.reshape(-1)), t, X, rows, cols).cpu().numpy()
+    bad = {3: (-1, np.inf), 8: (-2, -np.inf), 9: (-1, np.nan), 21: (0, np.inf), 36: (-1, -np.inf)}
+    for r, (block, scale) in bad.items():
+        w_np[r, block, :2] = np.array([scale], np.float16).view(np.uint8)
+    w = dev(cuda, w_np.reshape(-1))
+    got = _run(cuda, w, t, X, rows, cols).cpu().numpy()
+    one = _singles(cuda, w, t, X, rows, cols, range(n)).cpu().numpy()
+    np.testing.assert_array_equal(got, one)  # NaN at the same places
+    assert not np.isfinite(got[:, list(bad)]).any()
+    keep = [r for r in range(rows) if r not in bad]
+    np.testing.assert_array_equal(f32bits(got[:, keep]), f32bits(clean[:, keep]))
+
+
 # Chunks of 16 bytes: less than a stage of 8, a partial stage, a partial segment of 64, one segment, one
 # chunk past it; tiles of 32 and (from 256 workgroups) of 64.
 FLOAT_CASES = [(1, 8, 9), (33, 40, 9), (17, 384, 20), (48, 512, 33), (65, 520, 64), (40, 1536, 31), (1040, 384, 1030)]
