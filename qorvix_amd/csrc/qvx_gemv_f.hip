@@ -85,6 +85,12 @@ template <> struct SrcLoose<T_BF16> : SrcPlain<T_BF16> {
   static __device__ inline Raw load(const uint8_t* p, int l) { return ldu<uint4>(p + 16 * l); }
 };
 
+// Four codes less their offset, as signed bytes.
+template <int OFF>
+__device__ inline uint32_t less4(uint32_t q) {
+  return (q + (0x80u - OFF) * 0x01010101u) ^ 0x80808080u;
+}
+
 // The formats of 32-element blocks: codes q at byte kQ (8 bits: element e at kQ + e; 4 bits: low nibbles
 // elements 0..15, high 16..31), fifth bits at byte kH (-1: none), scale d at byte 0, offset m at byte 2
 // (kM) or a constant kOff subtracted from the code.
@@ -103,14 +109,21 @@ struct Src32 {
     r.dm = kM ? ldu<uint32_t>(b) : (uint32_t)ldu<uint16_t>(b);
     return r;
   }
+  // A value is the code's product with d, not a sum in which an infinite scale would meet its own opposite.
   static __device__ inline void widen(const Raw& r, float (&f)[8]) {
-    const float d = f16lo(r.dm), m = kM ? f16hi(r.dm) : -(float)kOff * d;
+    const float d = f16lo(r.dm), m = f16hi(r.dm);
+    uint32_t q[2] = {r.q.x, r.q.y};
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      if constexpr (!kByte) q[i] &= 0x0F0F0F0Fu;
+      if constexpr (kH >= 0) q[i] |= Lane<T_Q5_0>::spread4(r.h >> (4 * i));
+      if constexpr (kOff > 0) q[i] = less4<kOff>(q[i]);
+    }
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
-      const uint32_t w = k < 4 ? r.q.x >> (8 * k) : r.q.y >> (8 * k - 32);
-      int q = kByte ? (int)(int8_t)w : (int)(w & 15u);
-      if constexpr (kH >= 0) q |= (int)(((r.h >> k) & 1u) << 4);
-      f[k] = __builtin_fmaf((float)q, d, m);  // the product is exact: one rounding at most
+      const uint32_t b = q[k >> 2] >> (8 * (k & 3));
+      if constexpr (kM) f[k] = __builtin_fmaf((float)(b & 0xFFu), d, m);  // the product is exact: one rounding
+      else f[k] = (float)(int)(int8_t)b * d;
     }
   }
 };
@@ -172,12 +185,11 @@ template <> struct Src<T_Q6_K> {
     return r;
   }
   static __device__ inline void widen(const Raw& r, float (&f)[8]) {
-    const float ds = f16lo(r.d) * (float)(int)(int8_t)r.sc, m = -32.0f * ds;
-    const uint32_t q[2] = {(r.l.x & 0x0F0F0F0Fu) | ((r.h.x & 0x03030303u) << 4),
-                           (r.l.y & 0x0F0F0F0Fu) | ((r.h.y & 0x03030303u) << 4)};
+    const float ds = f16lo(r.d) * (float)(int)(int8_t)r.sc;
+    const uint32_t q[2] = {less4<32>((r.l.x & 0x0F0F0F0Fu) | ((r.h.x & 0x03030303u) << 4)),
+                           less4<32>((r.l.y & 0x0F0F0F0Fu) | ((r.h.y & 0x03030303u) << 4))};
 #pragma unroll
-    for (int k = 0; k < 8; ++k)  // ds (q - 32), rounded once
-      f[k] = __builtin_fmaf((float)((q[k >> 2] >> (8 * (k & 3))) & 0xFFu), ds, m);
+    for (int k = 0; k < 8; ++k) f[k] = (float)(int)(int8_t)(q[k >> 2] >> (8 * (k & 3))) * ds;
   }
 };
 

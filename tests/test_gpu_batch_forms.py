@@ -137,6 +137,37 @@ def test_loose_blocks(cuda, t, rows, cols, offset, n):
     _check(cuda, t, rows, cols, n, seed=rows + cols + n, bias=True, tol=FP32_TOL, offset=offset)
 
 
+# The formats whose values are a code (less an offset) times a scale: the block's bytes up to its codes, and the
+# whole block as bytes that make every value positive under a positive scale.
+POSITIVE = {qvx.Q8_0: (2, 5), qvx.Q8_1: (4, 5), qvx.Q4_0: (2, 0xFF), qvx.Q5_0: (2, 0xFF)}
+
+
+@pytest.mark.parametrize("t", [*POSITIVE, qvx.Q6_K])
+@pytest.mark.parametrize("n", [1, 3, 9])
+def test_loose_blocks_infinite_scales(cuda, t, n):
+    """An infinite scale over codes of one sign makes the outputs infinite, not NaN, on the fp32-activation
+    kernels: each value is its code times the scale, as the block formats define it."""
+    rng = np.random.default_rng(n)
+    rows, cols, offset = 40, 768, 2
+    w_np = random_weight(t, rows, cols, rng)
+    if t == qvx.Q6_K:
+        b = w_np.reshape(rows, 3, 210)
+        for r, sc in ((2, 1), (3, 0xFF)):  # scales +1 and -1
+            b[r, 1, :192], b[r, 1, 192:208] = 0xFF, sc
+            b[r, 1, 208:] = np.array([np.inf], np.float16).view(np.uint8)
+    else:
+        at, code = POSITIVE[t]
+        b = w_np.reshape(rows, cols // 32, -1)
+        for r, d in ((2, np.inf), (3, -np.inf)):
+            b[r, 5, at:] = code
+            b[r, 5, :2] = np.array([d], np.float16).view(np.uint8)
+    X_np = (np.abs(rng.standard_normal((n, cols))) + 0.1).astype(np.float32)
+    w = dev(cuda, np.concatenate([np.zeros(offset, np.uint8), w_np]))[offset:]
+    got = _run(cuda, w, t, dev(cuda, X_np), rows, cols).cpu().numpy()
+    assert (got[:, 2] == np.inf).all() and (got[:, 3] == -np.inf).all()
+    assert np.isfinite(np.delete(got, [2, 3], axis=1)).all()
+
+
 def test_loose_rows_past_the_staging_budget(cuda):
     """Rows of more than 32768 elements read their activations from global memory, four vectors a launch."""
     _check(cuda, qvx.Q4_1, 5, 33024, 7, seed=5, tol=2e-4)
