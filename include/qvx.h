@@ -109,6 +109,11 @@ int qvx_qmatmul(float* d_out, const void* d_w, uint32_t type, const float* d_x, 
  *   - once per 16 vectors: 9 to 32 vectors (23 on rows of < 2048 elements); 8 to 64 on up to 8192 rows of >=
  *     2048 elements; 5 to 64 on rows of >= 8192 elements (where rows of > 22528 elements take 8 a pass); with
  *     a norm or SwiGLU folded in (below) 6 to 256 on up to 8192 rows, from 8 or 9 on more;
+ *   - once per 8 or 16 vectors, each K range in a workgroup of its own: 5 to 16 vectors on fewer than 2048 rows
+ *     of >= 8192 elements (23 past 14336), and on up to 4096 rows past 22528 (the activations are not converted
+ *     beforehand then; the temporary holds rows/32 * KQ * 1 or 2 KiB of range sums, KQ = 4, 8 or 16);
+ *   - once per 16 or 64 vectors, the same range sums in the temporary: 25 to 32 vectors on up to 2048 rows of >=
+ *     14336 elements, 12 to 32 on more rows past 22528;
  *   - once per 64 vectors: larger batches -- the reference's "dequantize each block once for all nVec dot
  *     products" (qmatmul.hpp:24-32).
  * Smaller batches stream them once per 8 vectors (once per call up to 3) and allocate nothing, and so do, on

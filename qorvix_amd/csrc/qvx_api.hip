@@ -52,6 +52,9 @@ void launch_read16(const void* src, size_t n16, uint32_t* flag, hipStream_t s);
 bool qgemm_deq_supported(uint32_t t, const void* w, const uint16_t* X, int K, int N, size_t row_bytes);
 int q4k_plan_desc(int M, int N, int K, int cus, int* desc, int cap);
 bool gemv_q6s_route(int nvec, int rows, int cols, size_t row_bytes, size_t* ws_bytes);
+bool gemv_q4s_route(int nvec, int rows, int cols, size_t row_bytes, size_t* ws_bytes);
+bool launch_gemv_q4s(const void* w, const float* X, float* Y, const float* bias, int nvec, int rows, int cols,
+                     size_t row_bytes, void* ws, hipStream_t s);
 bool launch_gemv_q6s(const void* w, const float* X, float* Y, int nvec, int rows, int cols, size_t row_bytes,
                      void* ws, hipStream_t s, uint32_t* cnt);
 int gemv_q6s_counters(int nvec, int rows, int cols);
@@ -234,11 +237,31 @@ int gemv_unfused(float* out, const void* w, uint32_t type, const float* X, int n
   return rc;
 }
 
+// Rows so long that k_gemv_q4b serves 8 vectors a launch (the records of two vector tiles do not fit in LDS), or
+// nearly so where its workgroups are few or its rows many.
+inline bool q4_long(int rows, int cols) { return cols > (rows >= 4096 && rows < 8192 ? 22528 : 20480); }
+
+// Whether a Q4_K batch takes the form that splits the K ranges over workgroups (k_gemv_q4s), whose partial
+// sums a second launch adds: few rows of many elements, where k_gemv_q4b, which holds whole rows in a
+// workgroup, leaves the chip idle.  Measured on MI355X, graph-replayed, k_gemv_q4b's conversion included, it
+// against this form: 64 x 24576 at 5 vectors 17.3 against 8.9 us and at 23 40.5 against 22.5, 1024 x 14336 at 16 15.0
+// against 12.3, 1024 x 8192 at 5 10.0 against 9.6 but at 17 (two launches of this form) 18.0 against 22.7; 2048 x 8192
+// at 8 10.5 against 12.9; of the longest rows 2048 x 32768 at 16 46 against 28 and at 23 62 against 54.5, 4096 x 32768
+// at 16 52 against 45 but 4096 x 28672 at 17 0.74 times this form's time.  (On more than 4096 rows of that length
+// a K range is wider than this form takes.)
+inline bool q4s_batch(int nvec, int rows, int cols) {
+  if (nvec < 5 || nvec > 23 || cols < 8192) return false;
+  if (!q4_long(rows, cols)) return rows < 2048 && nvec <= (cols > 14336 ? 23 : 16);
+  return rows <= (nvec <= 16 ? 4096 : 2048);
+}
+
 // Whether a Q4_K batch takes the form on converted activations (k_gemv_q4b) rather than the many-vector form
 // or chunks of 8 on the one-vector / batched forms.  Its conversion is a launch of ~3 us (which a plan's
 // call on the activations of the call before it does without).  Measured on MI355X, graph-replayed over
 // distinct weights and activations, conversion included: on rows of >= 8192 elements from 5 vectors (4096 x
-// 14336 at 4: 17.7 against 19.1 us, at 5: 20.5 -> 19.1, at 16: 29.8 -> 24.2, at 64: 117 -> 67); from 8 on up to
+// 14336 at 4: 17.7 against 19.1 us, at 5: 20.5 -> 19.1, at 16: 29.8 -> 24.2, at 64: 117 -> 67; but the many-vector form,
+// whose K ranges lie on several workgroups up to 32 vectors, where rows are few and long, 64 x 24576 at 32 32.3 against
+// 51.9, or longest, 8192 x 24576 at 16 50 against 66, at 25 79 against 114, 9216 x 28672 at 64 279 against 342); from 8 on up to
 // 8192 rows of >= 2048 (4096 x 4096: 9.7 -> 9.1, 1024 x 4096: 9.4 -> 7.5; at 7 8.8 against 9); from 9 on others
 // (14336 x 4096 at 8 15.1 against 16, at 16: 23.7 -> 19.2; 8192 x 1024 at 9: 9.2 -> 7.8); to 64 where the
 // many-vector form's waves are few (4096 x 4096: 40.7 -> 28.6), to 32 on more rows (14336 x 4096 at 32: 36.4 ->
@@ -248,6 +271,12 @@ int gemv_unfused(float* out, const void* w, uint32_t type, const float* X, int n
 // 9 on others (11264 x 2048 at 8 10.9 against 11.6, at 9: 16.2 -> 13.2), and no many-vector form takes over.
 inline bool q4b_batch(int nvec, int rows, int cols, const GemvEpi& epi) {
   if (epi.flags()) return nvec >= (rows <= 8192 ? 6 : cols >= 4096 ? 8 : 9) && nvec <= 256;
+  if (q4_long(rows, cols)) {
+    if (rows > 4096) return (nvec >= 5 && nvec < 12) || (nvec > 32 && nvec <= (rows < 8192 ? 64 : 48));
+    if (nvec >= (rows <= 2048 ? 24 : 25) && nvec <= 32) return false;
+  } else if (rows <= 2048 && cols >= 14336 && nvec >= 25 && nvec <= 32) {
+    return false;
+  }
   if (cols >= 8192) return nvec >= 5 && nvec <= 64;
   if (cols < 2048) return nvec >= 9 && nvec <= 23;
   return rows <= 8192 ? nvec >= 8 && nvec <= 64 : nvec >= 9 && nvec <= 32;
@@ -275,7 +304,7 @@ inline bool q6_norm_batched(int nvec, int rows, int cols) {
 }
 
 // The forms that take a workspace, and the bytes of the one a call takes (0: none).
-enum WsForm { WS_NONE, WS_MANY, WS_Q6S, WS_Q6S_NORM, WS_INT, WS_Q4B };
+enum WsForm { WS_NONE, WS_MANY, WS_Q4S, WS_Q6S, WS_Q6S_NORM, WS_INT, WS_Q4B };
 inline WsForm ws_route(uint32_t type, int nvec, int rows, int cols, size_t row_bytes, bool fast, const GemvEpi& epi,
                        size_t* bytes) {
   *bytes = 0;
@@ -284,6 +313,9 @@ inline WsForm ws_route(uint32_t type, int nvec, int rows, int cols, size_t row_b
     *bytes = gemv_int_ws_bytes(type, nvec, rows, cols, row_bytes);
     if (*bytes) return WS_INT;
   }
+  if (type == T_Q4_K && !epi.flags() && q4s_batch(nvec, rows, cols) &&
+      gemv_q4s_route(nvec, rows, cols, row_bytes, bytes))
+    return WS_Q4S;
   if (type == T_Q4_K && q4b_batch(nvec, rows, cols, epi) && (epi.flags() == 0 || mx_epi_supported(epi, rows, cols))) {
     *bytes = gemv_q4b_ws_bytes(nvec, cols);
     if (*bytes) return WS_Q4B;
@@ -338,6 +370,8 @@ int gemv(float* out, const void* w, uint32_t type, const float* X, int nvec, int
   //  * Q4_K batches of 12-24 vectors or more (many_batch; encoder and prefill sizes): activations
   //    converted once, the weights streamed once per 64 vectors, bit-identical per vector to the
   //    one-vector kernel (k_gemv_q4k_many), with the bias added in its epilogue.
+  //  * Q4_K batches on few long rows (q4s_batch): the K ranges split over workgroups (k_gemv_q4s),
+  //    bit-identical per vector to the one-vector kernel, the bias added in its sum launch;
   //  * smaller Q4_K batches (q4b_batch): activations converted once, the batched form's tiles for 16 vectors
   //    a launch (k_gemv_q4b), bit-identical per vector to the one-vector kernel; a bias is added after; a
   //    capturing stream keeps the chunked forms where they are cheap (captured_temp);
@@ -365,6 +399,7 @@ int gemv(float* out, const void* w, uint32_t type, const float* X, int nvec, int
                              s, cnt);
       } else {
         ok = form == WS_MANY ? launch_gemv_q4k_many(w, X, out, epi.bias, nvec, rows, cols, row_bytes, ws, s)
+             : form == WS_Q4S ? launch_gemv_q4s(w, X, out, epi.bias, nvec, rows, cols, row_bytes, ws, s)
              : form == WS_Q4B ? launch_gemv_q4b(w, X, out, nvec, rows, cols, row_bytes, epi, ws, s)
              : form == WS_INT ? launch_gemv_int(type, w, X, out, epi.bias, nvec, rows, cols, row_bytes, ws, s)
                               : launch_gemv_q6s(w, X, out, nvec, rows, cols, row_bytes, ws, s, cnt);

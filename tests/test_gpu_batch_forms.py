@@ -275,6 +275,17 @@ def test_q4k_batches_match_single_vectors(cuda, rows, cols, n):
     _check(cuda, qvx.Q4_K, rows, cols, n, seed=rows + cols + n, bias=True, zero_vec=True)
 
 
+# Q4_K batches of few long rows, their K ranges split over workgroups (k_gemv_q4s): one row, ragged rows, one and
+# two items a wave, 8 and 16 vectors a launch, two launches, ranges of unequal length.
+Q4S_CASES = [(1, 8192, 5), (33, 8448, 8), (1000, 8192, 16), (70, 11264, 9), (515, 14336, 7), (64, 24576, 17),
+             (40, 20480, 23), (3000, 24576, 12), (2047, 32768, 16)]
+
+
+@pytest.mark.parametrize("rows,cols,n", Q4S_CASES)
+def test_q4k_batches_of_few_long_rows_match_single_vectors(cuda, rows, cols, n):
+    _check(cuda, qvx.Q4_K, rows, cols, n, seed=rows + cols + n, bias=True, zero_vec=True)
+
+
 @pytest.mark.parametrize("rows,cols,n", [(64, 512, 6), (320, 4096, 16), (96, 1024, 40), (9216, 1024, 9)])
 def test_q4k_batches_norm_and_swiglu_match_single_vectors(cuda, rows, cols, n):
     rng = np.random.default_rng(rows + n)
