@@ -106,9 +106,11 @@ int qvx_qmatmul(float* d_out, const void* d_w, uint32_t type, const float* d_x, 
  * Q4_K batches on the one-vector kernel's shapes (cols a multiple of 256 up to 32768, aligned operands)
  * convert the activations once into a stream-ordered temporary from the library's pool (nvec * cols * 2.25
  * bytes) and then stream the weights
- *   - once per 16 vectors: 9 to 32 vectors (23 on rows of < 2048 elements); 8 to 64 on up to 8192 rows of >=
- *     2048 elements; 5 to 64 on rows of >= 8192 elements (where rows of > 22528 elements take 8 a pass); with
- *     a norm or SwiGLU folded in (below) 6 to 256 on up to 8192 rows, from 8 or 9 on more;
+ *   - once per 16 vectors: 9 to 24 vectors (23 on rows of < 2048 elements; to 11 past 65536 rows); 8 to 64 on up to
+ *     8192 rows of more than 3072 elements (2048 on up to 4096 rows), to 48 on rows of >= 2048; 5 to 48 on rows of
+ *     >= 8192 elements (where rows of > 22528 elements take 8 a pass); 25 to 32 on more rows of >= 2048 where
+ *     16-row tiles fill 4/5 of a workgroup a CU; with a norm or SwiGLU folded in (below) 6 to 256 on up to 8192 rows
+ *     of >= 4096 elements, from 7, 8 or 9 on others;
  *   - once per 8 or 16 vectors, each K range in a workgroup of its own: 5 to 16 vectors on fewer than 2048 rows
  *     of >= 8192 elements (23 past 14336), and on up to 4096 rows past 22528 (the activations are not converted
  *     beforehand then; the temporary holds rows/32 * KQ * 1 or 2 KiB of range sums, KQ = 4, 8 or 16);

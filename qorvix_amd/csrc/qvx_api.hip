@@ -255,31 +255,56 @@ inline bool q4s_batch(int nvec, int rows, int cols) {
   return rows <= (nvec <= 16 ? 4096 : 2048);
 }
 
+// Whether the row tiles of the Q4_K geometry fill at least 4/5 of the places its workgroups have for them (one
+// workgroup a CU, a power of two of 16-row tiles at once).
+inline bool q4_filled(int rows) {
+  int64_t places = 4096;
+  while (places < rows) places += places < 65536 ? places : 65536;
+  return 5 * (int64_t)rows >= 4 * places;
+}
+
 // Whether a Q4_K batch takes the form on converted activations (k_gemv_q4b) rather than the many-vector form
 // or chunks of 8 on the one-vector / batched forms.  Its conversion is a launch of ~3 us (which a plan's
 // call on the activations of the call before it does without).  Measured on MI355X, graph-replayed over
-// distinct weights and activations, conversion included: on rows of >= 8192 elements from 5 vectors (4096 x
-// 14336 at 4: 17.7 against 19.1 us, at 5: 20.5 -> 19.1, at 16: 29.8 -> 24.2, at 64: 117 -> 67; but the many-vector form,
-// whose K ranges lie on several workgroups up to 32 vectors, where rows are few and long, 64 x 24576 at 32 32.3 against
-// 51.9, or longest, 8192 x 24576 at 16 50 against 66, at 25 79 against 114, 9216 x 28672 at 64 279 against 342); from 8 on up to
-// 8192 rows of >= 2048 (4096 x 4096: 9.7 -> 9.1, 1024 x 4096: 9.4 -> 7.5; at 7 8.8 against 9); from 9 on others
-// (14336 x 4096 at 8 15.1 against 16, at 16: 23.7 -> 19.2; 8192 x 1024 at 9: 9.2 -> 7.8); to 64 where the
-// many-vector form's waves are few (4096 x 4096: 40.7 -> 28.6), to 32 on more rows (14336 x 4096 at 32: 36.4 ->
-// 32.2, at 64 49 against 57) and to 23 on short rows (8192 x 1024 at 24 12.1 against 12.2).  With a norm or
-// SwiGLU folded in the batched form's conversion is longer: from 6 vectors on up to 8192 rows (6144 x 4096:
-// 13.8 -> 11.5), from 8 on more rows of >= 4096 (28672 x 4096 at 6 24.3 against 25.2, at 8: 26.7 -> 25.2), from
-// 9 on others (11264 x 2048 at 8 10.9 against 11.6, at 9: 16.2 -> 13.2), and no many-vector form takes over.
+// distinct weights and activations, conversion included:
+//  * to 8 vectors: from 5 on rows of >= 8192 elements (4096 x 14336 at 4: 17.7 against 19.1 us, at 5: 20.5 ->
+//    19.1), at 8 on up to 8192 rows longer than 2048 (3072 past 4096 rows) (4096 x 4096: 9.7 -> 9.1, 1024 x 4096:
+//    9.4 -> 7.5; at 7 8.8 against 9; 8192 x 2048 7.2 against 8.0);
+//  * 9 to 24 everywhere (14336 x 4096 at 16: 23.7 -> 19.2; 8192 x 1024 at 9: 9.2 -> 7.8), but at 24 rows of < 2048
+//    elements are equal (8192 x 1024 12.1 against 12.2); where 9 to 11 meet many short rows (65536 x 512 at 9 15.5 against
+//    14.1) and from 12 past 65536 rows, of which a CU's workgroups run one after another (70000 x 4096 at 16 100 against
+//    85, 128256 x 4096 at 25 211 against 176), the other forms;
+//  * 25 to 32 on up to 8192 rows of >= 2048 elements and where the rows fill the workgroups' places (14336 x 4096 at
+//    32: 36.4 -> 32.2; 11264 x 3072 0.88 times as fast, 20480 x 4096 0.95);
+//  * 33 to 48, three launches of 16 against the many-vector form's one of 64, whose waves are few: on up to 8192 rows
+//    (4096 x 4096 at 48 0.60 of its time) and on rows of >= 8192 elements (16384 x 8192 0.89);
+//  * 49 to 64 on up to 8192 rows longer than 2048 (3072 past 4096 rows) (4096 x 14336 at 64: 117 -> 67; 4096 x 4096: 40.7 ->
+//    28.6; but 8192 x 3072 1.22 times the other's time, 4096 x 2048 1.14, 16384 x 8192 1.14);
+//  * the many-vector form, whose K ranges lie on several workgroups up to 32 vectors, where rows are few and long, 64
+//    x 24576 at 32 32.3 against 51.9, or longest, 8192 x 24576 at 16 50 against 66, at 25 79 against 114, 9216 x 28672 at
+//    64 279 against 342.
+// With a norm or SwiGLU folded in the batched form's conversion is longer, and no many-vector form takes over: from 6
+// vectors on up to 8192 rows of >= 4096 elements (6144 x 4096: 13.8 -> 11.5), from 7 on up to 4096 of >= 2048 and 8
+// on up to 8192 of those (4096 x 2048 at 7 0.91 of its time; 8192 x 2048 at 6 1.08, at 8 0.96), from 8 on more rows of
+// >= 4096 (28672 x 4096 at 6 24.3 against 25.2, at 8: 26.7 -> 25.2), from 9 on others (4096 x 1024 at 8 1.11, 11264 x 2048
+// at 8 10.9 against 11.6, at 9: 16.2 -> 13.2).
 inline bool q4b_batch(int nvec, int rows, int cols, const GemvEpi& epi) {
-  if (epi.flags()) return nvec >= (rows <= 8192 ? 6 : cols >= 4096 ? 8 : 9) && nvec <= 256;
-  if (q4_long(rows, cols)) {
-    if (rows > 4096) return (nvec >= 5 && nvec < 12) || (nvec > 32 && nvec <= (rows < 8192 ? 64 : 48));
-    if (nvec >= (rows <= 2048 ? 24 : 25) && nvec <= 32) return false;
-  } else if (rows <= 2048 && cols >= 14336 && nvec >= 25 && nvec <= 32) {
-    return false;
+  if (epi.flags()) {
+    const int least = cols < 2048 ? 9 : rows > 8192 ? (cols >= 4096 ? 8 : 9) : cols >= 4096 ? 6 : rows <= 4096 ? 7 : 8;
+    return nvec >= least && nvec <= 256;
   }
-  if (cols >= 8192) return nvec >= 5 && nvec <= 64;
-  if (cols < 2048) return nvec >= 9 && nvec <= 23;
-  return rows <= 8192 ? nvec >= 8 && nvec <= 64 : nvec >= 9 && nvec <= 32;
+  if (nvec < 5 || nvec > 64) return false;
+  if (q4_long(rows, cols)) {
+    if (rows > 4096) return nvec < 12 || (nvec > 32 && nvec <= (rows < 8192 ? 64 : 48));
+    return nvec < (rows <= 2048 ? 24 : 25) || nvec > 32;
+  }
+  const bool wide = cols > (rows <= 4096 ? 2048 : 3072);
+  if (nvec <= 8) return cols >= 8192 || (nvec == 8 && rows <= 8192 && wide);
+  if (rows > 65536 && many_batch(nvec, rows, cols)) return false;
+  if (nvec <= 24) return cols >= 2048 || (nvec <= 23 && (nvec >= 12 || cols >= 1024 || rows <= 32768));
+  if (nvec <= 32) return cols >= 2048 && (rows > 8192 ? q4_filled(rows) : rows > 2048 || cols < 14336);
+  if (nvec <= 48) return cols >= 8192 || (rows <= 8192 && cols >= 2048);
+  return rows <= 8192 && wide;
 }
 
 // Whether a call that is being captured, with no workspace of its own, may put a temporary's allocation into
