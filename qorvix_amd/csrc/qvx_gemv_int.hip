@@ -13,9 +13,9 @@
 //  * the same reduction: a balanced pairwise tree over each 64 consecutive slots (over the next power of
 //    two, at least 8, for shorter rows), the 64-slot sums added in order.  The one-vector kernel's
 //    padding lanes add their mirrored last slot times 0: a zero of that slot's sign, or NaN where the
-//    slot's sum is not finite (a non-finite scale).  Here padding slots add -0, the same sum (a zero sum is
-//    -0 only where every slot's is, the last one's included), and a padded row's last slot adds its own
-//    sum times 0 to itself.
+//    slot's sum is not finite, which takes a non-finite scale.  Here padding slots add -0, the same sum (a
+//    zero sum is -0 only where every slot's is, the last one's included), and a padded row whose last
+//    slot's scales are not finite is NaN.
 #include "qvx_gemv_valu.hpp"
 
 namespace qvx {
@@ -34,6 +34,12 @@ typedef int i32x16_t __attribute__((ext_vector_type(16)));
 // elements 16g .. 16g + 15 of the slot's two 32-element blocks as signed bytes, and the block scales.
 // w = the slot's bytes in LDS (dword aligned).
 template <uint32_t T> struct IntFmt;
+// A zero where a slot's two scales are finite, else NaN.  p = the slot in memory (2-byte aligned).
+template <uint32_t T>
+__device__ inline float scales_zero(const uint8_t* p) {
+  const float d0 = f16lo(ldg2(p)), d1 = f16lo(ldg2(p + IntFmt<T>::kSlot / 2));
+  return __builtin_fmaf(d1, 0.0f, d0 * 0.0f);
+}
 template <> struct IntFmt<T_Q8_0> {
   static constexpr int kSlot = 68;
   static __device__ inline void codes(const uint32_t* w, int g, uint32_t (&c0)[4], uint32_t (&c1)[4], float& d0,
@@ -169,7 +175,6 @@ __global__ __launch_bounds__(64 * KS * VT, 2) void k_gemv_int(const uint8_t* __r
   // span / KS slots a wave, nck chunks a part.
   const int span = min(Sp, 64), part = span / KS, nck = part / kC, lck = 31 - __clz(nck), nblk = (S + span - 1) / span;
   const bool many = Sp > 64;
-  const int last = S - (S % span != 0 ? 1 : 0);  // a padded row's last slot, or none: the slots from it on need care
 
   // Copies chunk c (block c / nck) of every part into ring half h, all threads, without a branch: rows
   // and chunks are whole 16-byte pieces, pieces past the row repeat its last one (their slots add
@@ -215,6 +220,9 @@ __global__ __launch_bounds__(64 * KS * VT, 2) void k_gemv_int(const uint8_t* __r
     SB[u] = *reinterpret_cast<const float4*>(sb + s * 16 + 4);
   };
 
+  // The running sums in LDS for Q8_0, whose forms of four and eight K parts spill (0.97 of the time over the range of
+  // shapes; the 4- and 5-bit formats, which do not, take 1.02 times theirs).
+  constexpr bool kTotLds = T == T_Q8_0 && KS >= 4;
   float tot[8], st[4][8];
 #pragma unroll
   for (int k = 0; k < 8; ++k) tot[k] = 0.0f;
@@ -237,7 +245,7 @@ __global__ __launch_bounds__(64 * KS * VT, 2) void k_gemv_int(const uint8_t* __r
 #pragma unroll
     for (int u = 0; u < kC; ++u) {
       const int s = s0 + u;
-      float p[8], f[8];
+      float p[8];
       const i32x16_t zero = {};
       const i32x16_t C0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(
           A0[u], i32x4_t{(int)c0[0], (int)c0[1], (int)c0[2], (int)c0[3]}, zero, 0, 0, 0);
@@ -252,16 +260,11 @@ __global__ __launch_bounds__(64 * KS * VT, 2) void k_gemv_int(const uint8_t* __r
       for (int k = 0; k < 8; ++k) {  // vector 4 (k/2) + 2g + k%2: accumulators 2k (qh), 2k + 1 (ql)
         const int t0 = (int)(((uint32_t)C0[2 * k] << 7) + (uint32_t)C0[2 * k + 1]);
         const int t1 = (int)(((uint32_t)C1[2 * k] << 7) + (uint32_t)C1[2 * k + 1]);
-        f[k] = __builtin_fmaf(e1, (float)t1, e0 * (float)t0);
-        p[k] = f[k] * sx[k];
+        const float f = __builtin_fmaf(e1, (float)t1, e0 * (float)t0);
+        p[k] = f * sx[k];
         asm volatile("" : "+v"(p[k]));  // rounded before the tree adds it
+        if (s >= S) p[k] = -0.0f;
       }
-      if (s >= last)  // uniform
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-          p[k] = s == last && last < S ? __builtin_fmaf(f[k], 0.0f, p[k]) : -0.0f;
-          asm volatile("" : "+v"(p[k]));  // in the branch, not selected on every slot
-        }
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
         if (u == 0) v[k] = p[k];
@@ -314,7 +317,12 @@ __global__ __launch_bounds__(64 * KS * VT, 2) void k_gemv_int(const uint8_t* __r
           }
         }
       }
-      if (many) {
+      if constexpr (kTotLds) {
+        float* ps = psum + vtl * KS * 512 + lane;  // part 0's place: it is not stored
+        if (ks == 0)
+#pragma unroll
+          for (int k = 0; k < 8; ++k) ps[64 * k] = many ? (b > 0 ? ps[64 * k] : 0.0f) + v[k] : v[k];
+      } else if (many) {
 #pragma unroll
         for (int k = 0; k < 8; ++k) tot[k] += v[k];
       } else {
@@ -327,10 +335,23 @@ __global__ __launch_bounds__(64 * KS * VT, 2) void k_gemv_int(const uint8_t* __r
   const int r = r0 + ln;
   if (ks != 0 || vt >= nvt || r >= rows) return;
   const float bb = bias ? bias[r] : 0.0f;
+  if constexpr (kTotLds)
+#pragma unroll
+    for (int k = 0; k < 8; ++k) tot[k] = psum[vtl * KS * 512 + 64 * k + lane];
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
     const int vv = 16 * vt + 4 * (k >> 1) + 2 * g + (k & 1);
     if (vv < nvec) Y[(size_t)vv * rows + r] = bias ? tot[k] + bb : tot[k];
+  }
+  // A padded row whose last scales are not finite.  (Read again and stored over the sums, as the loop has no
+  // register to spare: with a NaN carried through it, or added to the sums, Q8_0 11008 x 4096 at 8 took 30.8 us, not 27.5.)
+  if (S % span != 0) {
+    const float pad = scales_zero<T>(wb + (size_t)ln * row_bytes + row_bytes - F::kSlot);
+    if (pad != pad)
+      for (int k = 0; k < 8; ++k) {
+        const int vv = 16 * vt + 4 * (k >> 1) + 2 * g + (k & 1);
+        if (vv < nvec) Y[(size_t)vv * rows + r] = pad;
+      }
   }
 }
 
