@@ -130,8 +130,10 @@ int qvx_qmatmul(float* d_out, const void* d_w, uint32_t type, const float* d_x, 
  * a workspace of its own, allocated by qvx_plan_instantiate, so its replays allocate nothing; on
  * shallow grids (<= 8 vectors, at most two 32-row tiles a workgroup) it also gives the call one
  * zeroed counter a 32-row tile, with which the kernel adds the block sums itself.
- * Q8_0 / Q4_0 / Q5_0 batches of 9 vectors or more (of 5 on weights of >= 32 Mi elements, 16 Mi for the 4-
- * and 5-bit formats), on the one-vector kernel's shapes, run on a matrix-core form that converts the
+ * Q8_0 / Q4_0 / Q5_0 batches of 9 vectors or more (Q8_0 of 11 to 17 on up to 2048 rows of >= 4096 elements, Q5_0
+ * of 11 on up to 1024 of >= 6144), Q4_0 and Q5_0 of 5 or more on weights of >= 16 Mi elements (past 8192 columns from
+ * 2048 or 4096 rows on) and Q8_0 of 7 or more on at least 4096 rows and 32 Mi elements (8 to 48 Mi up to 8192
+ * columns), on the one-vector kernel's shapes, run on a matrix-core form that converts the
  * activations once into a stream-ordered temporary (n_vec * cols * 2.06 bytes, at most about 64 MiB: larger
  * batches run in parts) or a plan's workspace, and reads the weights once per 16 to 64 vectors; on a
  * capturing stream they keep the one-vector kernel's launches, which take no temporary.

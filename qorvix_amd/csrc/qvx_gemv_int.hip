@@ -105,15 +105,34 @@ inline size_t int_ws_bytes(int nvec, int S) {
   const size_t nvt = ((size_t)nvec + 15) / 16;
   return nvt * S * (kFragBytes + 64);
 }
-// Whether a call takes this form rather than the VALU kernel, two or four vectors a launch.  Its fixed cost
-// (the conversion launch, the latency of a chunk's copies and of a wave's slots) is 7-15 us on short
-// weights, whatever the batch; measured on MI355X, graph-replayed over distinct weights: from 9 vectors it
-// is faster everywhere (4096 x 4096 at 12: Q8_0 23.6 -> 18.9 us, Q4_0 24.0 -> 12.8; 1024 x 4096 Q8_0 15.2 ->
-// 15.0), from 5 on weights of 16 Mi elements in the 4- and 5-bit formats (Q4_0 4096 x 4096 at 8: 16.1 ->
-// 12.6; 1024 x 4096: 10.7 against 11.1) and of 32 Mi in Q8_0 (11008 x 4096 at 8: 33.8 -> 27.5; 4096 x
-// 4096: 16.2 against 18.6).
+// Whether a call takes this form rather than the VALU kernel, which takes four vectors a launch, two or one for
+// the rest (5 vectors are two launches, 7 are three).  This form's time hardly depends on the batch, but grows with K
+// where its workgroups are few: a wave's K part is a serial chain.  Measured on MI355X, graph-replayed over distinct
+// weights, the VALU kernel against this form:
+//  * from 9 vectors it is faster on most shapes (4096 x 4096 at 12: Q8_0 23.6 -> 18.9 us, Q4_0 24.0 -> 12.8; 1024 x 4096
+//    Q8_0 at 12 15.2 -> 15.0), not on few long rows: Q8_0 1024 x 4096 at 9 14.5 against 15.5, 1024 x 8192 at 12 21.3
+//    against 23.9, 256 x 28672 at 12 56 against 65 and at 16 75 against 72, 2048 x 14336 at 9 1.16 times as long; Q5_0 256
+//    x 14336 at 9 1.07;
+//  * of 5 to 8, the 4- and 5-bit formats on weights of 16 Mi elements (Q4_0 4096 x 4096 at 8: 16.1 -> 12.6; 1024 x
+//    4096: 10.7 against 11.1), past 8192 columns only from 2048 rows on, 5 and 6 from 4096 (2048 x 14336 at 5 1.36
+//    times as long, 4096 x 14336 at 5 27.9 against 31.1 and at 6 equal);
+//  * Q8_0 at 7 and 8 (5 and 6 are two launches of the VALU kernel, the second a short one: 8192 x 6144 at 6 1.42 times
+//    as long) on 4096 rows and weights of 32 Mi elements (11008 x 4096 at 8: 33.8 -> 27.5), at 8 to 48 Mi where columns
+//    are no more than 8192 (32000 x 4096 at 7 0.87 of the time, at 8 1.07).
 inline bool int_batch(uint32_t t, int nvec, int rows, int cols) {
-  return nvec >= 9 || (nvec >= 5 && (int64_t)rows * cols >= ((int64_t)(t == T_Q8_0 ? 32 : 16) << 20));
+  const int64_t n = (int64_t)rows * cols, Mi = (int64_t)1 << 20;
+  if (t == T_Q8_0) {
+    if (nvec >= 9) {
+      const int least = cols < 4096 || rows > 2048 ? 9 : rows > 1024 || cols <= 4096 ? 11 : cols < 14336 ? 13 : 17;
+      return nvec >= least;
+    }
+    if (nvec < 7 || rows < 4096 || n < 32 * Mi) return false;
+    return cols > 8192 ? rows > 4096 || n < 48 * Mi : n < 48 * Mi || (nvec == 7 && rows > 8192);
+  }
+  if (nvec >= 9) return nvec >= 11 || t != T_Q5_0 || rows > 1024 || cols < 6144;
+  if (nvec < 5 || n < 16 * Mi) return false;
+  if (cols <= 8192) return true;
+  return rows >= (nvec <= 6 ? 4096 : 2048) && (nvec > 5 || rows > 4096 || cols < 14336);
 }
 // Vectors converted at a time: all of a call, or as many whole tiles as keep the workspace within 64 MiB.
 inline int int_chunk_vectors(int nvec, int S) {
