@@ -138,7 +138,7 @@ int qvx_qmatmul(float* d_out, const void* d_w, uint32_t type, const float* d_x, 
  * batches run in parts) or a plan's workspace, and reads the weights once per 16 to 64 vectors; on a
  * capturing stream they keep the one-vector kernel's launches, which take no temporary.
  * The fp32-activation kernels (see qvx_supports) read the weights once per 8 vectors from 9 vectors (from 5
- * on 8192 rows or more), per 4 below. */
+ * on 8192 rows or more, and on rows of up to 1024 elements), per 4 below. */
 int qvx_qmatmul_n(float* d_out, const void* d_w, uint32_t type, const float* d_X, int n_vec,
                   int rows, int cols, void* stream);
 

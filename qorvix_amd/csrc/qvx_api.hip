@@ -166,10 +166,11 @@ inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 // Whether a call runs on the fp32-activation kernels' tiled form, which adds the bias itself: a large
 // enough batch of unquantised weights in whole chunks, or of block weights that no integer kernel
 // takes (unaligned ones, and Q4_1 / Q5_1 / Q8_1).
-inline bool float_tiled(uint32_t type, int nvec, int rows, int cols, bool fast, const void* X) {
+inline bool float_tiled(uint32_t type, int nvec, int rows, int cols, bool fast, const void* w, const void* X) {
   if (!gemv_float_tiled(nvec, rows) || !aligned16(X)) return false;
   switch (type) {
-    case T_F32: case T_F16: case T_BF16: return fast && cols % (type == T_F32 ? 4 : 8) == 0 && cols <= 32768;
+    case T_F32: return cols % 8 == 0 ? (reinterpret_cast<uintptr_t>(w) & 3u) == 0 : fast && cols % 4 == 0 && cols <= 32768;
+    case T_F16: case T_BF16: return cols % 8 == 0;
     case T_Q4_1: case T_Q5_1: case T_Q8_1: return true;
     default: return !fast;
   }
@@ -435,7 +436,7 @@ int gemv(float* out, const void* w, uint32_t type, const float* X, int nvec, int
       return hip_status();
     }
   }
-  if (epi.bias && !float_tiled(type, nvec, rows, cols, fast, X)) {  // every other route: the plain product, then the bias add
+  if (epi.bias && !float_tiled(type, nvec, rows, cols, fast, w, X)) {  // every other route: the plain product, then the bias add
     GemvEpi plain = epi;
     plain.bias = nullptr;
     if (int rc = gemv(out, w, type, X, nvec, rows, cols, s, plain); rc != QVX_OK) return rc;

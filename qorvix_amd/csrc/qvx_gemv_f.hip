@@ -36,12 +36,13 @@ __device__ inline V ldu(const uint8_t* p) {
 
 // ---- weight chunks -----------------------------------------------------------------------------------
 // Src<T>: E elements a chunk; kU chunks a lane of the streaming form requests at a time; kSeg bytes a segment of
-// 64 chunks; Raw = a chunk's bytes in registers; load() issues its loads (chunk l of the segment at p: the
+// 64 chunks; kAligned = 16-byte aligned rows; Raw = a chunk's bytes in registers; load() issues its loads (chunk l of the segment at p: the
 // lane's part of the address is the same in every segment); widen() forms the fp32 values.
 template <uint32_t T> struct Src;
 
 template <uint32_t T> struct SrcPlain {  // 16 bytes of fp32 / fp16 / bf16 values
   static constexpr int E = T == T_F32 ? 4 : 8, kU = 8, kSeg = 1024;
+  static constexpr bool kAligned = true;
   typedef uint4 Raw;
   static __device__ inline Raw load(const uint8_t* p, int l) { return *reinterpret_cast<const uint4*>(p + 16 * l); }
   static __device__ inline void widen(const Raw& w, float (&f)[E]) {
@@ -67,6 +68,7 @@ template <> struct Src<T_BF16> : SrcPlain<T_BF16> {};
 // Unquantised weights at any alignment: 8 elements a chunk.
 template <uint32_t T> struct SrcLoose;
 template <> struct SrcLoose<T_F32> {
+  static constexpr bool kAligned = false;
   static constexpr int E = 8, kU = 4, kSeg = 2048;
   struct Raw { uint4 a, b; };
   static __device__ inline Raw load(const uint8_t* p, int l) {
@@ -79,9 +81,11 @@ template <> struct SrcLoose<T_F32> {
   }
 };
 template <> struct SrcLoose<T_F16> : SrcPlain<T_F16> {
+  static constexpr bool kAligned = false;
   static __device__ inline Raw load(const uint8_t* p, int l) { return ldu<uint4>(p + 16 * l); }
 };
 template <> struct SrcLoose<T_BF16> : SrcPlain<T_BF16> {
+  static constexpr bool kAligned = false;
   static __device__ inline Raw load(const uint8_t* p, int l) { return ldu<uint4>(p + 16 * l); }
 };
 
@@ -96,6 +100,7 @@ __device__ inline uint32_t less4(uint32_t q) {
 // (kM) or a constant kOff subtracted from the code.
 template <int BB, int kQ, bool kByte, int kH, bool kM, int kOff>
 struct Src32 {
+  static constexpr bool kAligned = false;
   static constexpr int E = 8, kU = 4, kSeg = 16 * BB;
   struct Raw { uint2 q; uint32_t h, dm; };
   static __device__ inline Raw load(const uint8_t* p, int l) {
@@ -137,6 +142,7 @@ template <> struct Src<T_Q5_1> : Src32<24, 8, false, 4, true, 0> {};
 // Q4_K / Q5_K: d, dmin and the 12 bytes of 6-bit scales and mins, Q5_K's fifth bits, the nibbles.
 template <bool kFive>
 struct SrcK45 {
+  static constexpr bool kAligned = false;
   static constexpr int E = 8, kU = 4, BB = kFive ? 176 : 144, kSeg = 2 * BB;
   struct Raw { uint4 hd; uint2 q, h; uint32_t j; };
   static __device__ inline Raw load(const uint8_t* p, int c) {
@@ -169,6 +175,7 @@ template <> struct Src<T_Q4_K> : SrcK45<false> {};
 template <> struct Src<T_Q5_K> : SrcK45<true> {};
 
 template <> struct Src<T_Q6_K> {
+  static constexpr bool kAligned = false;
   static constexpr int E = 8, kU = 4, kSeg = 420;
   struct Raw { uint2 l, h; uint32_t sc, d; };
   static __device__ inline Raw load(const uint8_t* p, int c) {
@@ -259,7 +266,7 @@ __global__ __launch_bounds__(1024) void k_gemv_float(const uint8_t* __restrict__
   request(w);
   bool fresh = true;  // w holds the block about to be summed
   if constexpr (STAGE) {
-    const int n4 = NV * cols / 4, per = cols / 4;
+    const int n4 = nv * cols / 4, per = cols / 4;
     for (int i = threadIdx.x; i < n4; i += (int)blockDim.x) {
       const int v = NV == 1 ? 0 : i / per, j = i - v * per;
       xs4[v * per + (j % XP) * nchunk + j / XP] = reinterpret_cast<const float4*>(X)[i];
@@ -427,8 +434,13 @@ bool launch_nv(const uint8_t* w, const float* X, float* Y, int rows, int cols, s
   const size_t lds = STAGE ? (size_t)NV * cols * 4 : 0;
   static LdsLimit lim;
   if (!lds_ready(reinterpret_cast<const void*>(kern), lim, lds)) return false;
-  // 16 waves a workgroup, 8 or 4 where that would leave CUs without one
-  const int nw = rows >= 16 * kCUs ? 16 : rows >= 8 * kCUs ? 8 : 4;
+  // 16 waves a workgroup, 8 or 4 where that would leave CUs without one, but not of aligned unquantised weights of
+  // 512 rows or more with much to stage, which 4 waves take longer over than the CUs save (fp16 1024 x 11008 at 2
+  // vectors 13.8 us with 4, 11.0 with 16, at 5888 columns 13.6 and 15 the other way; fp32 1024 x 5888 at 4 14.3 and 11.0, at 11008 and 2 16.7 and
+  // 19.5; Q6_K 64 x 11008 at 2 14.6 and 16.6).
+  const bool stage = S::kAligned && rows >= 2 * kCUs && rows < 8 * kCUs &&
+                     (S::E == 4 ? cols <= 8192 && lds >= 64 * 1024 : cols > 8192 && lds >= 80 * 1024);
+  const int nw = rows >= 16 * kCUs || stage ? 16 : rows >= 8 * kCUs ? 8 : 4;
   const int nwg = (int)std::min<int64_t>(kCUs, ((int64_t)rows + nw - 1) / nw);
   kern<<<(unsigned)nwg, (unsigned)(64 * nw), lds, s>>>(w, X, Y, rows, cols, row_bytes, nv);
   return true;
@@ -446,18 +458,25 @@ bool launch_src(const void* w, const float* X, float* Y, const float* bias, int 
                      rows, cols, row_bytes, s);
     return true;
   }
-  // vectors per launch: as many (1, 2 or 4) as the LDS budget stages, four unstaged ones otherwise
-  const size_t per = (size_t)cols * 4;
+  // vectors per launch: as many (4, 2 or 1) as the LDS budget stages, four unstaged ones otherwise; 3 and 5 to 8 too
+  // on rows of up to 1024 elements, whose launches are all ramp (see gemv_float_tiled; but fp16 256 x 2816 at 5 in one
+  // launch 9.3 us, in two 8.0).
+  const size_t fit = kLdsX / ((size_t)cols * 4);
   for (int v0 = 0; v0 < nvec;) {
-    const int left = nvec - v0;
+    const int left = nvec - v0, most = cols <= 1024 ? 8 : fit >= 4 || fit == 0 ? 4 : fit >= 2 ? 2 : 1;
+    const int nv = left == 3 && fit > 0 && cols > 1024 ? 2 : std::min(left, most);
     const float* Xv = X + (size_t)v0 * cols;
     float* Yv = Y + (size_t)v0 * rows;
     bool ok;
-    int nv;
-    if (4 * per <= kLdsX && left >= 4) ok = launch_nv<S, 4, true>(wb, Xv, Yv, rows, cols, row_bytes, nv = 4, s);
-    else if (2 * per <= kLdsX && left >= 2) ok = launch_nv<S, 2, true>(wb, Xv, Yv, rows, cols, row_bytes, nv = 2, s);
-    else if (per <= kLdsX) ok = launch_nv<S, 1, true>(wb, Xv, Yv, rows, cols, row_bytes, nv = 1, s);
-    else ok = launch_nv<S, 4, false>(wb, Xv, Yv, rows, cols, row_bytes, nv = std::min(4, left), s);
+    if (fit > 0)
+      ok = nv > 4    ? launch_nv<S, 8, true>(wb, Xv, Yv, rows, cols, row_bytes, nv, s)
+           : nv > 2  ? launch_nv<S, 4, true>(wb, Xv, Yv, rows, cols, row_bytes, nv, s)
+           : nv == 2 ? launch_nv<S, 2, true>(wb, Xv, Yv, rows, cols, row_bytes, nv, s)
+                     : launch_nv<S, 1, true>(wb, Xv, Yv, rows, cols, row_bytes, nv, s);
+    else
+      ok = nv > 2    ? launch_nv<S, 4, false>(wb, Xv, Yv, rows, cols, row_bytes, nv, s)
+           : nv == 2 ? launch_nv<S, 2, false>(wb, Xv, Yv, rows, cols, row_bytes, nv, s)
+                     : launch_nv<S, 1, false>(wb, Xv, Yv, rows, cols, row_bytes, nv, s);
     if (!ok) return false;
     v0 += nv;
   }
@@ -489,7 +508,7 @@ bool launch_gemv_float(uint32_t t, const void* w, const float* X, float* Y, cons
 }
 
 // GEMV over weights at any alignment, in chunks of 8 elements: cols % 8 == 0, X 16-byte aligned (and fp32
-// weights dword aligned).  Unquantised weights here always stream (bias must be null).
+// weights dword aligned).  bias only with a tiled call.
 bool launch_gemv_loose(uint32_t t, const void* w, const float* X, float* Y, const float* bias, int nvec, int rows,
                        int cols, size_t row_bytes, hipStream_t s) {
   if (cols % 8 != 0 || (reinterpret_cast<uintptr_t>(X) & 15u) != 0 ||
@@ -497,9 +516,9 @@ bool launch_gemv_loose(uint32_t t, const void* w, const float* X, float* Y, cons
     return false;
   const bool tiled = gemv_float_tiled(nvec, rows);
   switch (t) {
-    case T_F32: return launch_src<SrcLoose<T_F32>>(w, X, Y, nullptr, nvec, rows, cols, row_bytes, false, s);
-    case T_F16: return launch_src<SrcLoose<T_F16>>(w, X, Y, nullptr, nvec, rows, cols, row_bytes, false, s);
-    case T_BF16: return launch_src<SrcLoose<T_BF16>>(w, X, Y, nullptr, nvec, rows, cols, row_bytes, false, s);
+    case T_F32: return launch_src<SrcLoose<T_F32>>(w, X, Y, bias, nvec, rows, cols, row_bytes, tiled, s);
+    case T_F16: return launch_src<SrcLoose<T_F16>>(w, X, Y, bias, nvec, rows, cols, row_bytes, tiled, s);
+    case T_BF16: return launch_src<SrcLoose<T_BF16>>(w, X, Y, bias, nvec, rows, cols, row_bytes, tiled, s);
     case T_Q8_0: return launch_src<Src<T_Q8_0>>(w, X, Y, bias, nvec, rows, cols, row_bytes, tiled, s);
     case T_Q8_1: return launch_src<Src<T_Q8_1>>(w, X, Y, bias, nvec, rows, cols, row_bytes, tiled, s);
     case T_Q4_0: return launch_src<Src<T_Q4_0>>(w, X, Y, bias, nvec, rows, cols, row_bytes, tiled, s);

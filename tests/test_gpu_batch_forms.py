@@ -15,9 +15,10 @@ from test_gpu_kernels import dev, f32bits, random_weight
 pytestmark = pytest.mark.gpu
 
 GEMV_TOL = 1e-3
-# fp32 activations and exact weight values: an output is a chain of 8 FMAs, 6 tree adds and K / 512 segment
-# adds, so its error is at most (14 + K / 512) 2^-24 sum |w x|; with sum |w x| <= 0.4 sqrt(K) max |ref| for
-# these inputs and K <= 11008, 36 * 6e-8 * 42.
+# fp32 activations and exact weight values: a lane's sum is one chain of FMAs over its chunks, K / 64 of them, and
+# 6 tree adds follow, so an output's error is at most (K / 64 + 6) 2^-24 sum |w x|; sum |w x| <= 0.4 sqrt(K) max |ref|
+# for these inputs, so 178 * 6e-8 * 42 = 4.5e-4 of max |ref| at K = 11008.  Such a bound assumes that every rounding
+# errs the same way; they are held to a fifth of it.
 FP32_TOL = 9e-5
 
 
@@ -110,8 +111,8 @@ def test_int_batch_non_finite_scales(cuda, t, cols):
     np.testing.assert_array_equal(f32bits(got[:, keep]), f32bits(clean[:, keep]))
 
 
-# Chunks of 16 bytes: less than a stage of 8, a partial stage, a partial segment of 64, one segment, one
-# chunk past it; tiles of 32 and (from 256 workgroups) of 64.
+# Chunks of 16 bytes: less than a segment of 64, a partial one, one segment (fp16), one chunk past it, more than a
+# stage of two segments; rows and vectors around the tiles of 32 x 8.
 FLOAT_CASES = [(1, 8, 9), (33, 40, 9), (17, 384, 20), (48, 512, 33), (65, 520, 64), (40, 1536, 31), (1040, 384, 1030)]
 
 
@@ -168,9 +169,19 @@ def test_loose_blocks_infinite_scales(cuda, t, n):
     assert np.isfinite(np.delete(got, [2, 3], axis=1)).all()
 
 
-def test_loose_rows_past_the_staging_budget(cuda):
-    """Rows of more than 32768 elements read their activations from global memory, four vectors a launch."""
-    _check(cuda, qvx.Q4_1, 5, 33024, 7, seed=5, tol=2e-4)
+@pytest.mark.parametrize("t", [qvx.Q4_1, qvx.F16])
+@pytest.mark.parametrize("n", [1, 2, 3, 7])
+def test_loose_rows_past_the_staging_budget(cuda, t, n):
+    """Rows of more than 32768 elements read their activations from global memory, up to four vectors a launch."""
+    _check(cuda, t, 5, 33024, n, seed=5, tol=3e-4, bias=True)
+
+
+# Around the tiled form's lines (9 vectors; 5 on 8192 rows), and 3 and 5 to 8 vectors a launch on short rows.
+@pytest.mark.parametrize("t", [qvx.F16, qvx.Q4_1])
+@pytest.mark.parametrize("rows,cols,n", [(8191, 64, 5), (8192, 64, 5), (8193, 1056, 8), (700, 1024, 8), (65, 1024, 3),
+                                         (65, 1056, 3), (1, 64, 7), (4097, 256, 6), (513, 5888, 4)])
+def test_float_batch_lines(cuda, t, rows, cols, n):
+    _check(cuda, t, rows, cols, n, seed=rows + n, bias=True, tol=FP32_TOL)
 
 
 def test_unaligned_row_pitch_rmsnorm(cuda):
