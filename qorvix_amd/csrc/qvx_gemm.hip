@@ -1740,11 +1740,12 @@ struct Q4kPlan {
 // bf16, conversion of X included: 4096 x 4096 at M = 17 28.3 -> 18.4 us and at 201 31.9 -> 25.5 (8 splits), 1024
 // x 4096 at 201 28.6 -> 20.4, 4096 x 14336 at 201 53.2 -> 46.4; Q6_K 4096 x 14336 at 201 65.3 -> 59.  Of two
 // splits only while the tiles are few: 2048 x 1024 at M = 17 (8 tiles) 17.1 -> 13.3 us, at 400 (32) 19.8 -> 19.0,
-// but 14336 x 4096 at 201 (112) 46.1 against 46.7 and at 400 69.8 against 76.2.
-// The int8 kernel: 4096 x 4096 at M = 17 47 -> 32.5 us and at 128 48.5 -> 38.2 (8 and 8 splits), 4096 x 14336 at 201 99.5 ->
-// 80.8, 1024 x 4096 at 2048 67 -> 58.6; 14336 x 4096 at 512 (two splits of 224 tiles) keeps the one launch, 130.
-inline bool split_sum(int splits, int ntiles) { return splits > 2 || (splits == 2 && ntiles <= 64); }
-inline bool split_sum(const Q4kLaunch& L) { return split_sum(L.splits, L.ntiles); }
+// but at 600 (40) 20.4 against 21.6, at 800 (56) 21.7 against 24.3, 14336 x 4096 at 201 (112) 46.1 against 46.7.
+// The int8 kernel (to 64 tiles of two splits): 4096 x 4096 at M = 17 47 -> 32.5 us and at 128 48.5 -> 38.2 (8 and 8
+// splits), 4096 x 14336 at 201 99.5 -> 80.8, 1024 x 4096 at 2048 67 -> 58.6; 14336 x 4096 at 512 (two splits of 224
+// tiles) keeps the one launch, 130.
+inline bool split_sum(int splits, int ntiles, int most) { return splits > 2 || (splits == 2 && ntiles <= most); }
+inline bool split_sum(const Q4kLaunch& L) { return split_sum(L.splits, L.ntiles, 32); }
 void launch_split_sum(float* out, const float* part, int M, int N, const Q4kLaunch& L, hipStream_t s) {
   k_split_sum<<<dim3((unsigned)L.bm / 8, (unsigned)L.ntiles), 512, 0, s>>>(part, out, M, N, L.splits, L.tm.mt_a, L.bm);
 }
@@ -2121,7 +2122,7 @@ int launch_qgemm(float* out, const void* w, uint32_t t, const uint16_t* X, int M
     const size_t sbytes = (size_t)nsl * ntile * 4 * kI8BM * 4;
     if (sbytes >= (1u << 31)) return -7;
     const size_t pbytes = splits > 1 ? (size_t)tiles * splits * kI8BM * kBN * 4 : 0;
-    const bool sum = split_sum(splits, tiles);
+    const bool sum = split_sum(splits, tiles, 64);
     const size_t cbytes = splits > 1 && !sum ? (((size_t)tiles * 4 + 255) & ~(size_t)255) : 0;
     uint8_t* qb = static_cast<uint8_t*>(gemm_ws(qbytes + sbytes + pbytes + cbytes, ws, ws_cap, s));
     if (!qb) return no_mem;
