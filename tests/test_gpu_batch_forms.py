@@ -57,11 +57,12 @@ def _check(torch, t, rows, cols, n, seed, bias=False, zero_vec=False, tol=GEMV_T
         np.testing.assert_array_equal(f32bits(gb.cpu().numpy()), f32bits((got + b).cpu().numpy()))
 
 
-# Slots of 64 elements: one slot; a short row's padded tree (6 of 8, 20 of 32); exactly one 64-slot block;
-# one slot past it; several blocks with a partial last one.  Rows: one, ragged, whole tiles.  Vectors: the
-# fewest (9, or 5 on large weights), one tile, one past it, several workgroups; few waves take the K parts,
-# many do not.
-INT_CASES = [(1, 64, 9), (4, 512, 12), (36, 2560, 16), (4200, 4096, 5), (8200, 4096, 7), (1, 64, 17), (33, 384, 20), (40, 1280, 33), (64, 4096, 17), (70, 4096, 65), (31, 4160, 18),
+# Slots of 64 elements: a short row's padded tree (4 of 8, 12 of 16, 20 of 32, 40 of 64); exactly one 64-slot block;
+# four slots past it; several blocks with a partial last one.  (A row of 1, 6 or 65 slots is no multiple of 16 bytes: those
+# cases run on the fp32-activation kernels.)  Rows: one, ragged, whole tiles.  Vectors: the fewest (9, or 5 or 7 on large
+# weights), one tile, one past it, several workgroups; few waves take the K parts, many do not.
+INT_CASES = [(3, 256, 9), (33, 768, 20), (31, 4352, 18), (8200, 4096, 8), (5000, 14336, 6), (5000, 14336, 8),
+             (1, 64, 9), (4, 512, 12), (36, 2560, 16), (4200, 4096, 5), (8200, 4096, 7), (1, 64, 17), (33, 384, 20), (40, 1280, 33), (64, 4096, 17), (70, 4096, 65), (31, 4160, 18),
              (100, 11008, 24), (1030, 4096, 70), (2080, 1024, 130), (1100, 4096, 260)]
 
 
@@ -69,6 +70,31 @@ INT_CASES = [(1, 64, 9), (4, 512, 12), (36, 2560, 16), (4200, 4096, 5), (8200, 4
 @pytest.mark.parametrize("rows,cols,n", INT_CASES)
 def test_int_batches_match_single_vectors(cuda, t, rows, cols, n):
     _check(cuda, t, rows, cols, n, seed=rows + cols + n, bias=True, zero_vec=True)
+
+
+def test_int_batch_in_parts(cuda):
+    """A batch whose converted activations pass the workspace's bound runs in parts of 992 vectors (32768 columns), the
+    last one ragged: bit-identical to single vectors around the parts' edge, eagerly with a bias and in a plan."""
+    from qorvix_amd import decode
+    rng = np.random.default_rng(9)
+    t, rows, cols, n = qvx.Q4_0, 33, 32768, 1003
+    w = dev(cuda, random_weight(t, rows, cols, rng))
+    X = cuda.randn(n, cols, device="cuda", generator=cuda.Generator(device="cuda").manual_seed(1))
+    bias = dev(cuda, rng.standard_normal(rows).astype(np.float32))
+    which = [0, 15, 16, 990, 991, 992, 993, 1001, 1002]
+    one = _singles(cuda, w, t, X, rows, cols, which)
+    got = _run(cuda, w, t, X, rows, cols, bias)
+    np.testing.assert_array_equal(f32bits(got[which].cpu().numpy()), f32bits((one + bias).cpu().numpy()))
+    out = cuda.empty((n, rows), dtype=cuda.float32, device="cuda")
+    plan = decode.Plan()
+    plan.add(out, decode.DevWeight(w, t, rows, cols), X, n)
+    plan.instantiate()
+    for _ in range(3):
+        out.fill_(float("nan"))
+        plan.launch(cuda.cuda.current_stream().cuda_stream)
+        cuda.cuda.synchronize()
+        np.testing.assert_array_equal(f32bits(out[which].cpu().numpy()), f32bits(one.cpu().numpy()))
+    plan.close()
 
 
 def test_int_batch_keeps_non_finite_vectors_apart(cuda):
@@ -341,14 +367,52 @@ def test_plan_batches_share_only_unchanged_activations(cuda):
     plan.close()
 
 
-# K splits of the prefill GEMM whose partial tiles a launch of their own sums (k_split_sum): 2, 4, 5, 7, 8 and 28
-# splits, a last split shorter than the others, subtiles and rows past M, columns past N.
-@pytest.mark.parametrize("t,M,rows,cols", [(qvx.Q4_K, 17, 2048, 1024), (qvx.Q4_K, 257, 4096, 14336),
-                                           (qvx.Q4_K, 65, 3300, 3328), (qvx.Q4_K, 201, 1001, 4096),
-                                           (qvx.Q4_K, 1, 256, 2304), (qvx.Q6_K, 17, 4096, 14336),
-                                           (qvx.Q6_K, 130, 1001, 4096), (qvx.Q6_K, 97, 300, 512)])
+@pytest.mark.parametrize("n", [1, 9])
+def test_plan_shares_norms_only_as_recorded(cuda, n):
+    """Consecutive calls on one x with a norm folded in share their conversion (batches) or a launch (one vector),
+    unless the norm weight or eps differs, or a call before writes the norm weight."""
+    from qorvix_amd import decode
+    rng = np.random.default_rng(n)
+    d = 512
+    w = [decode.DevWeight(dev(cuda, random_weight(qvx.Q4_K, d, d, rng, scale=1e-3)), qvx.Q4_K, d, d) for _ in range(3)]
+    x = dev(cuda, rng.standard_normal((n, d)).astype(np.float32))
+    na0, nb = (dev(cuda, (1 + 0.1 * rng.standard_normal(d)).astype(np.float32)) for _ in range(2))
+    buf = cuda.empty(n * d, dtype=cuda.float32, device="cuda")  # an output whose first row is a norm weight
+    na = buf[:d]
+    outs = [cuda.zeros((n, d), dtype=cuda.float32, device="cuda") for _ in range(6)]
+    steps = [(outs[0], w[0], na, 1e-5), (outs[1], w[1], na, 1e-5), (outs[2], w[0], nb, 1e-5), (outs[3], w[0], nb, 1e-1),
+             (buf.view(n, d), w[2], nb, 1e-1), (outs[4], w[1], na, 1e-5), (outs[5], w[0], na, 1e-5)]
+    plan = decode.Plan()
+    for o, ww, nw, eps in steps:
+        plan.add_rmsnorm(o, ww, x, nw, eps, n)
+    plan.instantiate()
+    call = lambda ww, nw, eps: qvx.qmatmul_rmsnorm_t(ww.data, ww.type, x, nw, eps, d, d)  # noqa: E731
+    written = call(w[2], nb, 1e-1)
+    want = [call(w[0], na0, 1e-5), call(w[1], na0, 1e-5), call(w[0], nb, 1e-5), call(w[0], nb, 1e-1),
+            call(w[1], written[0].contiguous(), 1e-5), call(w[0], written[0].contiguous(), 1e-5)]
+    st = cuda.cuda.current_stream().cuda_stream
+    for run in (plan.launch, plan.launch, plan.run_eager):
+        na.copy_(na0)
+        run(st)
+        cuda.cuda.synchronize()
+        for o, e in zip(outs, want):
+            np.testing.assert_array_equal(f32bits(o.cpu().numpy()), f32bits(e.cpu().numpy()))
+    plan.close()
+
+
+# K splits of the prefill GEMM whose partial tiles a launch of their own sums (k_split_sum): a last split shorter than
+# the others, subtiles and rows past M, columns past N.  splits: as planned for 256 CUs (0: Q6_K, not exposed; 14, 8
+# and 4 by the same rule).
+@pytest.mark.parametrize("t,M,rows,cols,splits", [(qvx.Q4_K, 17, 2048, 1024, 4), (qvx.Q4_K, 257, 4096, 14336, 5),
+                                                  (qvx.Q4_K, 65, 3300, 3328, 7), (qvx.Q4_K, 201, 1001, 4096, 8),
+                                                  (qvx.Q4_K, 1, 256, 2304, 5), (qvx.Q4_K, 128, 6144, 1024, 2),
+                                                  (qvx.Q4_K, 130, 3000, 1024, 2), (qvx.Q6_K, 17, 4096, 14336, 0),
+                                                  (qvx.Q6_K, 130, 1001, 4096, 0), (qvx.Q6_K, 97, 300, 2048, 0)])
 @pytest.mark.parametrize("variant", [qvx.GEMM_BF16, qvx.GEMM_F16])
-def test_gemm_k_split_sum(cuda, t, M, rows, cols, variant):
+def test_gemm_k_split_sum(cuda, t, M, rows, cols, splits, variant):
+    if splits:
+        plan = qvx.qgemm_plan_q4k(M, rows, cols, 256)
+        assert plan[0]["splits"] == splits and (splits > 2 or plan[0]["tiles"] <= 32)
     rng = np.random.default_rng(M + rows)
     w = dev(cuda, random_weight(t, rows, cols, rng, scale=1e-3))
     X = dev(cuda, (0.5 * rng.standard_normal((M, cols))).astype(np.float16))

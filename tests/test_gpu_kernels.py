@@ -495,12 +495,11 @@ def test_gemm_split_k_overwrites_stale_output(cuda, variant, offset):
 @pytest.mark.parametrize("t,variant", [(qvx.Q4_K, qvx.GEMM_BF16), (qvx.Q4_K, qvx.GEMM_F16), (qvx.Q4_K, qvx.GEMM_I8),
                                        (qvx.Q6_K, qvx.GEMM_BF16), (qvx.Q6_K, qvx.GEMM_F16)])
 @pytest.mark.parametrize("M,rows,cols", [(128, 14336, 4096), (37, 2048, 4096), (300, 4096, 14336)])
-def test_gemm_split_k_is_deterministic(cuda, t, variant, M, rows, cols):
-    """Shapes whose grid is smaller than the chip split K; the split that finishes a tile last adds
-    the partial tiles in split order 0, 1, ..., so repeated calls (whichever split finishes first)
-    give the same bits, and the result stays within the GEMM tolerance of the fp64 oracle on a
-    slice of rows (bf16 / fp16 variants)."""
-    if t == qvx.Q4_K:
+def test_gemm_split_k_is_deterministic(cuda, t, variant, M, rows, cols, splits=True):
+    """Shapes whose grid is smaller than the chip split K; the partial tiles are added in split order 0, 1, ...
+    (here by a launch of their own), so repeated calls give the same bits, and the result stays within the GEMM
+    tolerance of the fp64 oracle on a slice of rows (bf16 / fp16 variants)."""
+    if t == qvx.Q4_K and splits:
         plan = qvx.qgemm_plan_q4k(M, rows, cols)
         assert variant == qvx.GEMM_I8 or plan[0]["splits"] > 1
     W = qvx.empty_weight(t, rows, cols)
@@ -516,6 +515,22 @@ def test_gemm_split_k_is_deterministic(cuda, t, variant, M, rows, cols):
     ref = X.cpu().numpy().astype(np.float64) @ Wd.reshape(len(idx), cols).astype(np.float64).T
     if variant != qvx.GEMM_I8:  # the Q8 arithmetic has its own oracle test
         assert max_rel(runs[0][:, idx], ref) <= GEMM_TOL
+
+
+# Two K splits of more than 32 tiles: the split that finishes a tile last adds the partial tiles (the int8 kernel's
+# from 65 tiles on).
+LAST_SPLIT_CASES = [(qvx.Q4_K, qvx.GEMM_BF16, 201, 14336, 4096), (qvx.Q4_K, qvx.GEMM_F16, 256, 14336, 4096),
+                    (qvx.Q4_K, qvx.GEMM_F16, 800, 2048, 1024), (qvx.Q6_K, qvx.GEMM_F16, 600, 4096, 2048),
+                    (qvx.Q6_K, qvx.GEMM_BF16, 600, 4096, 2048), (qvx.Q4_K, qvx.GEMM_I8, 512, 14336, 4096)]
+
+
+@pytest.mark.parametrize("t,variant,M,rows,cols", LAST_SPLIT_CASES)
+def test_gemm_last_split_sums_are_deterministic(cuda, t, variant, M, rows, cols):
+    """The same bits whichever split finishes first, within the GEMM tolerance of the fp64 oracle on a slice of rows."""
+    if t == qvx.Q4_K and variant != qvx.GEMM_I8:
+        plan = qvx.qgemm_plan_q4k(M, rows, cols, 256)
+        assert plan[0]["splits"] == 2 and plan[0]["tiles"] > 32
+    test_gemm_split_k_is_deterministic(cuda, t, variant, M, rows, cols, splits=False)
 
 
 @pytest.mark.parametrize("t", [qvx.Q4_K, qvx.Q6_K])
@@ -555,14 +570,14 @@ def test_gemm_split_k_concurrent_streams(cuda, t):
 def test_gemm_split_k_counters_reused_across_calls(cuda):
     """Calls that may allocate take their K split's tile counters from a block the stream keeps,
     cleared once: every launch leaves the counters it used at zero.  K-split calls of different
-    tile counts and kernels (the Q4_K and Q6_K raw-block GEMMs, the 16-bit GEMM behind Q8_0 / Q4_0),
-    fp16 and bf16, interleaved on one stream for three rounds and then on a new stream, give the
+    tile counts and kernels (the Q4_K and Q6_K raw-block GEMMs at two splits of more than 32 tiles, the 16-bit GEMM
+    behind Q8_0 / Q4_0; and raw-block calls that use none), fp16 and bf16, interleaved on one stream for three rounds and then on a new stream, give the
     first round's bits every time (a counter left non-zero would make a later tile's last split
     skip its sum, or sum too early)."""
     cases = [(qvx.Q4_K, qvx.GEMM_F16, 128, 14336, 4096), (qvx.Q6_K, qvx.GEMM_F16, 300, 4096, 14336),
              (qvx.Q4_K, qvx.GEMM_BF16, 37, 2048, 4096), (qvx.Q8_0, qvx.GEMM_BF16, 128, 4096, 4096),
              (qvx.Q4_K, qvx.GEMM_F16, 200, 1024, 4096), (qvx.Q6_K, qvx.GEMM_BF16, 128, 1024, 4096),
-             (qvx.Q4_0, qvx.GEMM_F16, 96, 4096, 11008)]
+             (qvx.Q4_0, qvx.GEMM_F16, 96, 4096, 11008)] + [c for c in LAST_SPLIT_CASES if c[1] != qvx.GEMM_I8]
     lib = qvx.lib()
     data = []
     for i, (t, variant, M, rows, cols) in enumerate(cases):

@@ -3,9 +3,9 @@ bias epilogue (qvx_qmatmul_n_bias, the reference's wmatmulNBias).
 
 The reference promises that qmatmulN is bit-identical to qmatmul per vector
 (runtime/include/qorvix/runtime/qmatmul.hpp:31-32).  The many-vector form converts the activations
-once and streams the weights once per 64 vectors (once per 16, with the K ranges split over
-workgroups, up to 32 vectors; it takes batches from 12 vectors on weights of >= 32 Mi elements and
-from 24 on smaller ones); these tests hold every output to the one-vector call's bits
+once and streams the weights once per 64 vectors (once per 16, with the K ranges split over waves and
+workgroups, up to 32 vectors); smaller and middling batches take k_gemv_q4b on converted activations, or
+k_gemv_q4s on few long rows.  These tests hold every output to the one-vector call's bits
 (qvx_qmatmul), and to the chunked batched forms' (calls of 8 vectors), at shapes whose one-vector
 geometry walks K in 1, 4 and 16 ranges (including the backward walks of even ranges), with ragged
 rows and vector counts on both sides of 32 and not multiples of 16 or 64.  A plan replays the
@@ -58,7 +58,12 @@ def _chunked(cuda, W, t, X, rows, cols):
 @pytest.mark.parametrize("rows,cols,nvec", [(14336, 4096, 64), (4096, 14336, 100), (1000, 4096, 37),
                                             (1024, 2048, 24), (300, 768, 130), (4096, 14336, 16),
                                             (14336, 4096, 12), (14336, 4096, 29), (128256, 4096, 20),
-                                            (4096, 4096, 32)])
+                                            (4096, 4096, 32),
+                                            # the many-vector form's shapes of up to 32 vectors, its K ranges in two
+                                            # workgroups, then in 8, 4, 2 and 1 waves of one
+                                            (300, 256, 24), (40, 768, 32), (33, 1792, 28), (64, 32768, 32),
+                                            (6000, 1024, 25), (5000, 24576, 12), (12000, 1024, 32), (20000, 1024, 24),
+                                            (40000, 512, 30), (70000, 768, 13)])
 def test_many_bit_identical_to_single_vector_calls(cuda, rows, cols, nvec):
     t = qvx.Q4_K
     W = _weight(cuda, t, rows, cols, seed=rows + nvec)
@@ -76,10 +81,11 @@ def test_many_bit_identical_to_single_vector_calls(cuda, rows, cols, nvec):
 
 
 def test_plan_replays_many_vector_calls(cuda):
-    """A plan's many-vector calls (in order, and two in one fork, which need disjoint workspace
-    slices) replay bit-identically to the direct calls, several times with eager work between."""
+    """A plan's batches (in order, and several in one fork, which need disjoint workspace slices) replay
+    bit-identically to the direct calls, several times with eager work between: converted activations, 64 vectors a
+    pass, and K ranges in two workgroups, whose partial sums and counters lie in the workspace."""
     t = qvx.Q4_K
-    shapes = [(4096, 14336, 16), (14336, 4096, 48), (4096, 4096, 24)]
+    shapes = [(4096, 14336, 16), (14336, 4096, 48), (4096, 4096, 24), (300, 768, 28), (64, 24576, 28)]
     Ws = [_weight(cuda, t, r, c, seed=40 + i) for i, (r, c, n) in enumerate(shapes)]
     Xs = [qvx.fill_normal_t(cuda.empty((n, c), dtype=cuda.float32, device="cuda"), seed=50 + i)
           for i, (r, c, n) in enumerate(shapes)]
@@ -88,7 +94,7 @@ def test_plan_replays_many_vector_calls(cuda):
     plan = decode.Plan()
     plan.add(outs[0], decode.DevWeight(Ws[0], t, *shapes[0][:2]), Xs[0], shapes[0][2])
     plan.fork()
-    for i in (1, 2):
+    for i in (1, 2, 3, 4):
         plan.add(outs[i], decode.DevWeight(Ws[i], t, *shapes[i][:2]), Xs[i], shapes[i][2])
     plan.join()
     plan.instantiate()
@@ -98,23 +104,23 @@ def test_plan_replays_many_vector_calls(cuda):
             o.fill_(float("nan"))
         plan.launch(s)
         cuda.cuda.synchronize()
-        for i in range(3):
+        for i in range(len(shapes)):
             assert cuda.equal(outs[i].view(cuda.int32), want[i].view(cuda.int32)), (rep, i)
     plan.close()
 
 
 def test_plan_replays_split_q4k_calls(cuda):
-    """The split Q4_K form in a plan (range partials in the plan's workspace, with a bias on one call):
-    replays bit-identical to the direct calls, several times."""
+    """Q4_K batches in a plan on converted activations and on the split form (few long rows, range partials in
+    the plan's workspace): replays bit-identical to the direct calls, several times."""
     t = qvx.Q4_K
-    shapes = [(4096, 14336, 8), (1024, 4096, 16)]
+    shapes = [(4096, 14336, 8), (1024, 4096, 16), (1024, 14336, 8), (70, 24576, 20)]
     Ws = [_weight(cuda, t, r, c, seed=80 + i) for i, (r, c, n) in enumerate(shapes)]
     Xs = [qvx.fill_normal_t(cuda.empty((n, c), dtype=cuda.float32, device="cuda"), seed=90 + i)
           for i, (r, c, n) in enumerate(shapes)]
     want = [_many(cuda, W, t, X, r, c) for W, X, (r, c, n) in zip(Ws, Xs, shapes)]
     outs = [cuda.full((n, r), float("nan"), dtype=cuda.float32, device="cuda") for (r, c, n) in shapes]
     plan = decode.Plan()
-    for i in range(2):
+    for i in range(len(shapes)):
         plan.add(outs[i], decode.DevWeight(Ws[i], t, *shapes[i][:2]), Xs[i], shapes[i][2])
     plan.instantiate()
     s = cuda.cuda.current_stream().cuda_stream
@@ -123,7 +129,7 @@ def test_plan_replays_split_q4k_calls(cuda):
             o.fill_(float("nan"))
         plan.launch(s)
         cuda.cuda.synchronize()
-        for i in range(2):
+        for i in range(len(shapes)):
             assert cuda.equal(outs[i].view(cuda.int32), want[i].view(cuda.int32)), (rep, i)
     plan.close()
 
@@ -202,10 +208,13 @@ def test_many_matches_oracle_at_encoder_batch(cuda):
 
 @pytest.mark.parametrize("t,rows,cols,nvec", [(qvx.Q4_K, 1000, 4096, 40), (qvx.Q4_K, 512, 4096, 3),
                                               (qvx.Q4_K, 700, 14336, 8), (qvx.Q6_K, 512, 4096, 20),
-                                              (qvx.F16, 300, 512, 5)])
+                                              (qvx.F16, 300, 512, 5), (qvx.Q4_K, 300, 768, 130),
+                                              (qvx.Q4_K, 14336, 4096, 64), (qvx.Q4_K, 300, 768, 28),
+                                              (qvx.Q4_K, 12000, 1024, 25), (qvx.Q4_K, 64, 24576, 28),
+                                              (qvx.Q4_K, 1024, 14336, 8)])
 def test_bias_is_one_add_after_the_product(cuda, t, rows, cols, nvec):
-    """qvx_qmatmul_n_bias == qvx_qmatmul_n + bias, bit for bit, on the many-vector form (its epilogue),
-    the split Q4_K form (its sum launch) and on the routes that add the bias in a launch of its own; a
+    """qvx_qmatmul_n_bias == qvx_qmatmul_n + bias, bit for bit, on the many-vector form (its epilogue, with
+    and without K ranges in several workgroups), the split Q4_K form (its sum launch) and on the routes that add the bias in a launch of its own; a
     null bias is qvx_qmatmul_n."""
     if t == qvx.F16:
         W = cuda.randn(rows * cols, device="cuda").to(cuda.float16).view(cuda.uint8)
