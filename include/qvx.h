@@ -22,8 +22,8 @@
  *  - Device entry points take device pointers and a hipStream_t passed as `void*` (NULL = the
  *    null stream).  They are asynchronous and stream-ordered, like the CUDA backend's matmulS
  *    launch (cuda/src/cuda_backend.cu:1534-1542).  They allocate no device memory, except
- *    qvx_qgemm_f16, qvx_gemm16, the many-vector forms of qvx_qmatmul_n and the unfused norm route,
- *    which take stream-ordered temporaries (the converted activations, the partial tiles of a K
+ *    qvx_qgemm_f16, qvx_gemm16, the many-vector forms of qvx_qmatmul_n, those of Q4_K and Q6_K batches with a
+ *    norm or SwiGLU folded in (qvx_qmatmul_n_rmsnorm, qvx_qmatmul_swiglu) and the unfused norm route, which take stream-ordered temporaries (the converted activations, the partial tiles of a K
  *    split, or the dequantised weight) from a memory pool the library owns per device.  Each stream
  *    keeps its last temporary for its next call (no pool call between back-to-back calls), and a
  *    block of K-split tile counters (64 KiB or more, cleared once, left zero by every launch) for
@@ -190,7 +190,10 @@ int qvx_qmatmul_group(float* const* d_out, const void* const* d_w, const uint32_
  * qvx_qmatmul_n plus d_norm_w [cols] (NULL -> QVX_E_NULL; cols > 16384 -> QVX_E_RANGE).  Where the GEMV kernel takes the shape
  * (Q4_K and the integer-dot formats, cols a multiple of 512 up to 16384, aligned operands) the norm
  * is folded into the kernel's activation conversion: one launch, no temporary; the per-vector
- * arithmetic does not depend on n_vec, so batches are bit-identical to single vectors.  Q6_K
+ * arithmetic does not depend on n_vec, so batches are bit-identical to single vectors.  Q4_K batches of 6 to 9
+ * vectors or more convert the normalised activations once, in a launch of its own, into a stream-ordered
+ * temporary (n_vec * cols * 2.25 bytes); on a capturing stream, or without the memory, they keep the one launch per
+ * 8 vectors.  Q6_K
  * batches the batched matrix-core form takes (cols a multiple of 2048; weights of >= 8192 rows or
  * columns, or 6 vectors or more) run the standalone norm into a stream-ordered temporary (n_vec *
  * cols * 4 bytes beside the form's block sums) and then that form: the norm forms the same bits as
@@ -204,7 +207,8 @@ int qvx_qmatmul_n_rmsnorm(float* d_out, const void* d_w, uint32_t type, const fl
  * (rows 32k .. 32k+15 = gate rows 16k .., rows 32k+16 .. 32k+31 = up rows 16k ..; build it with
  * qvx_interleave_rows16), 2 * ffn rows; out [n_vec, ffn].  ffn % 16 != 0 -> QVX_E_SHAPE.  Q4_K with
  * ffn % 16 == 0 and aligned operands runs fused (the gate and up tiles of a workgroup meet in its
- * epilogue); other calls run the product into a temporary and a standalone SwiGLU. */
+ * epilogue; batches of 6 to 9 vectors or more take the temporary that qvx_qmatmul_n_rmsnorm's do); other calls
+ * run the product into a temporary and a standalone SwiGLU. */
 int qvx_qmatmul_swiglu(float* d_out, const void* d_w_gu, uint32_t type, const float* d_X,
                        const float* d_norm_w, float eps, int n_vec, int ffn, int cols, void* stream);
 /* Interleave two [rows, cols] weights of `type` in 16-row groups into d_dst (2 rows x cols), the

@@ -176,7 +176,8 @@ inline bool float_tiled(uint32_t type, int nvec, int rows, int cols, bool fast, 
   }
 }
 
-// Whether a Q4_K batch takes the many-vector form rather than chunks of 8 vectors.  The form costs
+// Whether a Q4_K batch that neither k_gemv_q4s nor k_gemv_q4b takes (below; asked first) runs on the many-vector
+// form rather than in chunks of 8 vectors.  The form costs
 // a conversion launch and a K-range chain per wave whatever the batch (17-22 us in graph replays on
 // MI355X), against ~10 us per 8-vector chunk of a 4096 x 4096 weight and 14-26 us of a 58.7 M-element
 // one: measured, it wins from 12 vectors on weights of >= 32 Mi elements (14336 x 4096 at 12: 20.2
@@ -393,7 +394,7 @@ int gemv(float* out, const void* w, uint32_t type, const float* X, int nvec, int
   // Forms with a workspace, which is the caller's (a plan sizes one at instantiation) or a
   // stream-ordered temporary; a call that may not allocate and has no workspace keeps the forms
   // below.
-  //  * Q4_K batches of 12-24 vectors or more (many_batch; encoder and prefill sizes): activations
+  //  * larger Q4_K batches, and some of 12 to 32 vectors (many_batch; encoder and prefill sizes): activations
   //    converted once, the weights streamed once per 64 vectors, bit-identical per vector to the
   //    one-vector kernel (k_gemv_q4k_many), with the bias added in its epilogue.
   //  * Q4_K batches on few long rows (q4s_batch): the K ranges split over workgroups (k_gemv_q4s),

@@ -325,7 +325,8 @@ __global__ __launch_bounds__(1024) void k_gemv_float(const uint8_t* __restrict__
 // activations and weights are requested before a stage is summed.  At the end the 32 sums of 64 lanes meet in
 // 8 registers: permlane swaps add two sums at a time over xor 32 and 16 (lanes 16 q .. 16 q + 15 then hold
 // sums 8 (q % 2) + 16 (q / 2) + j), DPP adds the rest -- the butterfly's own pairs.
-// Bound by the FMAs; the LDS reads that feed them take half their time.  Measured on MI355X, graph-replayed:
+// Of a 384-wide encoder's launches VALU instructions fill 0.21 of the cycles and waves wait 0.47 of theirs: short rows leave
+// half of a stage empty, and ramp, the first stage's loads and the butterfly are most of a launch.  Measured on MI355X, graph-replayed:
 // fp16 384 x 1536 at 256 vectors 12.6 us, where 64 launches of the streaming form took 290; 14336 x 4096 at
 // 16 vectors 110 -> 57 us; Q6_K 32000 x 3072 at 16 570 -> 114 us (the byte-by-byte decode this file's block
 // chunks replaced; its one-vector call 126 -> 43, 2048 x 5632 24 -> 7.8).
@@ -459,8 +460,8 @@ bool launch_src(const void* w, const float* X, float* Y, const float* bias, int 
     return true;
   }
   // vectors per launch: as many (4, 2 or 1) as the LDS budget stages, four unstaged ones otherwise; 3 and 5 to 8 too
-  // on rows of up to 1024 elements, whose launches are all ramp (see gemv_float_tiled; but fp16 256 x 2816 at 5 in one
-  // launch 9.3 us, in two 8.0).
+  // on rows of up to 1024 elements, whose launches are all ramp (Q6_K 1024 x 256 at 5 7.3 -> 4.9 us, at 7, three launches,
+  // 10.3 -> 4.9; but fp16 256 x 2816 at 5 in one launch 9.3 us, in two 8.0).
   const size_t fit = kLdsX / ((size_t)cols * 4);
   for (int v0 = 0; v0 < nvec;) {
     const int left = nvec - v0, most = cols <= 1024 ? 8 : fit >= 4 || fit == 0 ? 4 : fit >= 2 ? 2 : 1;

@@ -165,8 +165,9 @@ __global__ __launch_bounds__(256) void k_int_conv(const float* __restrict__ X, i
 // and the parts -- whole subtrees -- are added through LDS.  The 32 rows' bytes of the next kC slots of
 // every part are copied into one half of an LDS ring while the other half is folded, so the weights are
 // read from memory once per VT * 16 vectors.
-// Bound by the fold (8 VALU instructions per row, vector and slot of some 110 a wave issues; the two MFMAs
-// of a slot take a fifth of its time) and by how the tiles divide over the SIMDs.  Measured on MI355X: 577
+// The fold is 8 VALU instructions per row, vector and slot of some 110 a wave issues, but over an encoder layer's launches
+// (577 x 1024, Q8_0) VALU instructions fill 0.19 of the SIMDs' cycles and MFMAs 0.03: the 320 workgroups of a 1024-row
+// weight lie unevenly on 256 CUs, one or two waves a SIMD, and each wave is a chain of chunks.  Measured on MI355X: 577
 // vectors of 1024 on 1024 rows of Q8_0, 12.6 us beside a 4.8 us conversion, where 145 launches of the
 // one-vector kernel took 580; 4096 rows 31 us; 4096 x 4096 at 64 vectors 121 -> 26 us with the conversion.
 template <uint32_t T, int KS, int VT>

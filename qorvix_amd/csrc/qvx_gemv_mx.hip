@@ -903,9 +903,9 @@ constexpr size_t kLdsMax = kLdsPerCU;
 // memory (L2): a wave reads the 512 bytes a sub-block and 8 vectors one super-block ahead of their use,
 // each register quad requested again as soon as its MFMAs are issued, so LDS holds only the records
 // (copied once a workgroup, 512 bytes a super-block and 8 vectors) and the tile ring, whatever K, and one
-// pass over the weights serves 16 vectors.  Bound by the fold's VALU work, ~185 instructions a tile, wave and
-// super-block at 8 vectors (the 15-bit products' scales, minimums and float sums, whose order is fixed), not
-// by memory.  Measured on MI355X, graph-replayed over distinct weights, without the conversion's ~3 us: 4096 x
+// pass over the weights serves 16 vectors.  The fold is ~185 instructions a tile, wave and super-block at 8 vectors (the
+// 15-bit products' scales, minimums and float sums, whose order is fixed), which fill 0.37 of the cycles of 14336 x 4096
+// at 16 vectors; waves wait 0.47 of theirs, for fragments and tiles: latency at 4 waves a SIMD, more than issue.  Measured on MI355X, graph-replayed over distinct weights, without the conversion's ~3 us: 4096 x
 // 4096 5.7 us at 8 vectors and 6.9 at 16 (9.4 and 18.5 on the forms that convert in every workgroup), 14336 x
 // 4096 12.3 and 16.2 (14.1 and 23.4 on the batched and the many-vector form), 4096 x 14336 13.0 and 17.4 (20.8
 // and 29.2 with the K ranges split over workgroups and summed by a second launch), 1024 x 4096 4.8 and 5.8 (9.1
