@@ -1800,8 +1800,9 @@ inline int cdiv(int a, int b) { return (a + b - 1) / b; }
 // workgroups costs 4 us and 1 us a slice, the sum 2 us, 0.6 us a split and the partials' write and read at 6
 // TB/s.  Measured on MI355X, bf16, conversion of X included: 4096 x 4096 at M = 257 with 8 splits (384 workgroups)
 // 34.2 us, with 4 28.6; 4096 x 14336 at 257 with 8 72.5, with 5 60.5; 2048 x 1024 at 17 with 2 13.3, with 4 10.9; Q6_K
-// 1024 x 4096 at 201 with 4 29.2, with 8 23.7, with 16 24.7; but 4096 x 4096 at 17 with 8 18.5, with 16 20.4.  More splits than `fewest` allows only where the partials (at
-// most 256 tiles, 32 MiB) fit the no-allocation scratch beside any copy of X.
+// 1024 x 4096 at 201 with 4 29.2, with 8 23.7, with 16 24.7; but 4096 x 4096 at 17 with 8 18.5, with 16 20.4.  More splits
+// than `fewest` allows only where the partials (at most 256 tiles, 32 MiB) fit the no-allocation scratch beside any copy
+// of X.
 int split_count(int M, int N, int nsl, int tiles, int fewest, int cus) {
   auto most = [&](int least) {
     int n = 1;
